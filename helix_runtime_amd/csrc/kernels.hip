@@ -472,6 +472,7 @@ struct DecodeKernelArgs {
   // folded into qscale).
   float k_scale;
   float v_scale;
+  int rows_aligned;  // query and tail rows are 16-byte aligned (stream mode, bf16 / fp8 pages)
 };
 
 __device__ __forceinline__ int clamp_length(int hist, int max_blocks) {
@@ -916,18 +917,10 @@ struct PageDesc {
 // global store after the last load.  A full stage is flushed early (many
 // short units per wavefront).
 constexpr int kStreamStage = 4;
-// fp8 stream wavefronts: four per SIMD with a one-deep result stage (the
-// extra wavefront hides more per-page latency than its spills cost).
-constexpr int kFp8StreamWaves = 4;
-constexpr int kFp8StreamStage = 1;
-
-
 // One token row's 4 dims of a page buffer as fp32: fp32 pages as loaded,
 // bf16 pages (4 per 64-bit lane load) widened where the row is used, so a
 // buffer never holds a widened copy of its page.
 __device__ __forceinline__ float4 page_row(const float4& x) { return x; }
-// First word of an fp8 page buffer row (the LDS query path orders on it).
-__device__ __forceinline__ unsigned first_word(const unsigned& x) { return x; }
 __device__ __forceinline__ float4 page_row(const uint2& x) { return bf16_widen(x.x, x.y); }
 __device__ __forceinline__ float4 page_row(const unsigned& x) { return fp8_widen4(x, 1.0f); }
 __device__ __forceinline__ float4 masked_row(const float4& x, bool keep) {
@@ -962,10 +955,9 @@ struct StreamShared {
 // them to separate __shared__ arrays: as distinct objects they are known not
 // to overlap, which the dynamically indexed fields of one struct are not
 // (the struct form cost 70 extra LDS reads and spills in the loop).
-// S: results staged before a flush.  qslot: query rows loaded straight
-// into LDS, one area per page buffer (reduced-precision pages), or null.
-template <int G, int S = kStreamStage>
+template <int G>
 struct StreamLds {
+  static constexpr int S = kStreamStage;  // results staged before a flush
   float (&p)[2][8 * G];
   float (&head)[3][G];
   float4 (&res_o)[S][G][32];
@@ -976,27 +968,11 @@ struct StreamLds {
   float4 (&app_k)[S][32];
   float4 (&app_v)[S][32];
   long long (&app_dst)[S];
-  float4 (*qslot)[G][32];
 };
 template <int G>
 __device__ __forceinline__ StreamLds<G> stream_lds(StreamShared<G>& s) {
   return StreamLds<G>{s.p, s.head, s.res_o, s.res_ml, s.res_dst,
-                      s.seg, s.seg_unit, s.app_k, s.app_v, s.app_dst, nullptr};
-}
-
-// fp8 pages in the stream kernel: query rows loaded straight into LDS (three
-// areas used by units in turn) and read from there at every page, with no register
-// copy; one result staged; four wavefronts per SIMD, which their small page
-// buffers then allow (119-127 VGPRs, at most 2 spilled).  Config 3, one
-// box: 104.0 us per layer against 108.5 with a register copy per unit
-// (6-13 spilled), 116.3 with three wavefronts and two staged results and
-// 140.4 with two wavefronts.  bf16 pages stay at two wavefronts: with the
-// same arrangement three ran 128.4-128.8 against 125.4 us (161 VGPRs, no
-// spills) and four 161.6 us (21-27 spilled).
-constexpr bool stream_lds_query_type(PageType t) { return t == PageType::kFP8; }
-template <int PF, int G>
-constexpr bool stream_lds_query() {
-  return G <= 4 && stream_lds_query_type(static_cast<PageType>(PF));
+                      s.seg, s.seg_unit, s.app_k, s.app_v, s.app_dst};
 }
 
 // LDS hand-off inside one wavefront.  In the stream kernel a workgroup is a
@@ -1016,12 +992,12 @@ __device__ __forceinline__ void stream_sync() {
 
 // The body of one stream wavefront: `wave` is its index among
 // a.stream_waves, `lane` its lane, `sh` its LDS.
-template <int G, bool APPEND, int PF, bool SHARED_BLOCK, int S = kStreamStage>
+template <int G, bool APPEND, int PF, bool SHARED_BLOCK>
 __device__ __forceinline__ void decode_stream_body(
     DecodeKernelArgs a, const std::uint32_t* __restrict__ tables,
     const std::int32_t* __restrict__ lengths, float* __restrict__ out,
     float* __restrict__ part_o, float* __restrict__ part_ml, int* __restrict__ segments,
-    const std::int64_t* __restrict__ append_slots, int wave, int lane, StreamLds<G, S> sh) {
+    const std::int64_t* __restrict__ append_slots, int wave, int lane, StreamLds<G> sh) {
   // The block table and lengths are read-only here and do not alias the
   // outputs; with the restrict-qualified parameters their uniform reads
   // become scalar loads.
@@ -1037,8 +1013,7 @@ __device__ __forceinline__ void decode_stream_body(
   constexpr int R = G >= 4 ? G / 4 : 1;
   constexpr int DUPB = G >= 4 ? 0 : (G == 2 ? 1 : 2);
   constexpr int NV = 8 * G;
-  constexpr int kStage = S;
-  constexpr bool QLDS = !SHARED_BLOCK && stream_lds_query<PF, G>();
+  constexpr int kStage = kStreamStage;
   // fp8 and bf16 pages, and stream wavefronts beside prefix workgroups: the
   // raw exp2 and a ballot for the rescale test (measured: config 3 fp8
   // 110.7 -> 108.4 us per layer, config 4 fused cascade 79.9 -> 79.3 us;
@@ -1178,20 +1153,7 @@ __device__ __forceinline__ void decode_stream_body(
   const int lane_off = lane * (FP8 ? 4 : BF16 ? 8 : 16);
   const int row_off = j * 16;
   using Raw = std::conditional_t<FP8, unsigned, std::conditional_t<BF16, uint2, float4>>;
-  // Query rows through LDS: a unit's rows go to area (kvh * batch + b) % 3.
-  // Units are visited in that flat order, every unit has a page (its
-  // tail) and loads run two pages ahead, so the unit that reuses an area
-  // (three units later) starts loading at least one page after the last
-  // read of the area's previous rows.  (Two areas would already reload an
-  // area only after its last read in program order; the third adds a page
-  // of margin.)
-  auto query_area = [&](const PageDesc& d) {
-    return static_cast<int>(
-        static_cast<unsigned>(__builtin_amdgcn_readfirstlane(d.kvh * a.batch + d.b)) % 3u);
-  };
-  // slot: the page buffer (0 or 1).
-  auto load_page = [&](const PageDesc& d, Raw (&k)[8], Raw (&v)[8], float4 (&q)[G], bool& bad,
-                       int slot) {
+  auto load_page = [&](const PageDesc& d, Raw (&k)[8], Raw (&v)[8], float4 (&q)[G], bool& bad) {
     const int b = __builtin_amdgcn_readfirstlane(d.b);
     const int kvh = __builtin_amdgcn_readfirstlane(d.kvh);
     const int p = __builtin_amdgcn_readfirstlane(d.p);
@@ -1224,24 +1186,10 @@ __device__ __forceinline__ void decode_stream_body(
     }
     if (p == 0 || d.g == g0) {
       const float* qsrc = a.query + (static_cast<std::size_t>(b) * a.q_heads + kvh * G) * D;
-      if constexpr (QLDS) {
-        // The G rows (G * 32 vectors of 16 bytes) straight into this
-        // buffer's LDS area, issued ahead of the page: the wait for the
-        // page's first key load covers them.
+      const __amdgpu_buffer_rsrc_t qr = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<float*>(qsrc), 0, d.skip ? 0 : G * D * 4, kBufferWord3);
 #pragma unroll
-        for (int i = 0; i < (G * 32 + 63) / 64; ++i) {
-          if (i * 64 + lane < G * 32) {
-            prefill_detail::lds_load16(qsrc + (i * 64 + lane) * 4,
-                                       prefill_detail::lds_address(&sh.qslot[query_area(d)][0][0]) +
-                                           i * 1024);
-          }
-        }
-      } else {
-        const __amdgpu_buffer_rsrc_t qr = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<float*>(qsrc), 0, d.skip ? 0 : G * D * 4, kBufferWord3);
-#pragma unroll
-        for (int h = 0; h < G; ++h) q[h] = as_float4(__builtin_amdgcn_raw_buffer_load_b128(qr, row_off, h * D * 4, 0));
-      }
+      for (int h = 0; h < G; ++h) q[h] = as_float4(__builtin_amdgcn_raw_buffer_load_b128(qr, row_off, h * D * 4, 0));
     }
     // A skip descriptor (past the end of the range) gets an empty buffer
     // range: its loads return zeros without touching memory, and the step
@@ -1500,17 +1448,14 @@ __device__ __forceinline__ void decode_stream_body(
   };
 
   float4 qc[G];  // query rows of the unit being processed
-  auto step_body = [&](const PageDesc& d, const auto& k, auto& v, const float4 (&qn)[G], int slot,
-                       bool bad) {
+  auto step_body = [&](const PageDesc& d, const auto& k, auto& v, const float4 (&qn)[G], bool bad) {
     int valid = 0;
     if (!d.skip) {
       valid = d.p == d.np - 1 ? 1 : min(P, d.hist - (d.p + a.first_page) * P);
       unit_bad = unit_bad || bad;
-      if constexpr (!QLDS) {
-        if (d.p == 0 || d.g == g0) {
+      if (d.p == 0 || d.g == g0) {
 #pragma unroll
-          for (int h = 0; h < G; ++h) qc[h] = qn[h];
-        }
+        for (int h = 0; h < G; ++h) qc[h] = qn[h];
       }
       if (d.p == 0) {
         // This wavefront holds the unit's first page: record which
@@ -1540,25 +1485,10 @@ __device__ __forceinline__ void decode_stream_body(
         stream_sync<SHARED_BLOCK>();
       }
     }
-    if constexpr (QLDS) {
-      // The query rows are read from the unit's LDS area at every page, so
-      // no register copy lives across the unit's pages.  The index depends
-      // (through an empty asm) on the page's first key word, so the read
-      // waits for that load, which was issued after the unit's query loads.
-      int dep = 0;
-      asm volatile("" : "+v"(dep) : "v"(first_word(k[0])));
-      float4 qv[G];
-      const int qa = query_area(d);
-#pragma unroll
-      for (int h = 0; h < G; ++h) qv[h] = sh.qslot[qa][h][j + dep];
-      process(k, v, qv, valid);
-    } else {
-      process(k, v, qc, valid);
-    }
+    process(k, v, qc, valid);
     if (!d.skip && (d.p == d.np - 1 || d.g == g1 - 1)) finalize(d);
   };
-  auto step = [&](const PageDesc& d, Raw (&kr)[8], Raw (&vr)[8], const float4 (&qn)[G], bool bad,
-                  int slot) {
+  auto step = [&](const PageDesc& d, Raw (&kr)[8], Raw (&vr)[8], const float4 (&qn)[G], bool bad) {
     if constexpr (FP8) {
       if (!d.skip && d.p == d.np - 1) {
         // The tail row arrived as fp32 in slots 0-3: its codes (the values
@@ -1580,62 +1510,46 @@ __device__ __forceinline__ void decode_stream_body(
                            bf16_pack(__uint_as_float(vr[1].x), __uint_as_float(vr[1].y)));
       }
     }
-    step_body(d, kr, vr, qn, slot, bad);
+    step_body(d, kr, vr, qn, bad);
   };
 
-  // Two pages in flight, each in its own register buffer.  More did not
-  // help the reduced-precision pages, whose kernels are held by their
-  // per-page instruction latency at two wavefronts per SIMD: bf16 with 3
-  // pages 130 against 125 us per config-3 layer (query rows moved to LDS to
-  // fit the registers), with 4 pages 191 us (LDS-limited occupancy); fp8
-  // with 3 and 4 pages 146 and 150 against 140 us.
+  // Two pages in flight, each in its own register buffer.
   Raw ka[8], va[8], kb[8], vb[8];
   bool bada, badb;
-  if constexpr (QLDS) {
+  float4 qa[G], qb[G];
 #pragma unroll
-    for (int h = 0; h < G; ++h) qc[h] = make_float4(0.f, 0.f, 0.f, 0.f);
-    PageDesc da = next_desc();
-    load_page(da, ka, va, qc, bada, 0);
-    PageDesc db = next_desc();
-    load_page(db, kb, vb, qc, badb, 1);
-    for (long long g = g0; g < g1; g += 2) {
-      step(da, ka, va, qc, bada, 0);
-      da = next_desc();
-      load_page(da, ka, va, qc, bada, 0);
-      step(db, kb, vb, qc, badb, 1);
-      db = next_desc();
-      load_page(db, kb, vb, qc, badb, 1);
-    }
-  } else {
-    float4 qa[G], qb[G];
-#pragma unroll
-    for (int h = 0; h < G; ++h) qa[h] = qb[h] = qc[h] = make_float4(0.f, 0.f, 0.f, 0.f);
-    PageDesc da = next_desc();
-    load_page(da, ka, va, qa, bada, 0);
-    PageDesc db = next_desc();
-    load_page(db, kb, vb, qb, badb, 1);
-    for (long long g = g0; g < g1; g += 2) {
-      step(da, ka, va, qa, bada, 0);
-      da = next_desc();
-      load_page(da, ka, va, qa, bada, 0);
-      step(db, kb, vb, qb, badb, 1);
-      db = next_desc();
-      load_page(db, kb, vb, qb, badb, 1);
-    }
+  for (int h = 0; h < G; ++h) qa[h] = qb[h] = qc[h] = make_float4(0.f, 0.f, 0.f, 0.f);
+  PageDesc da = next_desc();
+  load_page(da, ka, va, qa, bada);
+  PageDesc db = next_desc();
+  load_page(db, kb, vb, qb, badb);
+  for (long long g = g0; g < g1; g += 2) {
+    step(da, ka, va, qa, bada);
+    da = next_desc();
+    load_page(da, ka, va, qa, bada);
+    step(db, kb, vb, qb, badb);
+    db = next_desc();
+    load_page(db, kb, vb, qb, badb);
   }
   flush();
 }
 
-template <int G, bool APPEND, int PF>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(
-    G > 4 ? 1 : (stream_lds_query<PF, G>() ? kFp8StreamWaves : 2))))
+}  // namespace
+}  // namespace helix::hip
+
+#include "decode_mma.hpp"
+
+namespace helix::hip {
+namespace {
+
+template <int G, bool APPEND>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(G > 4 ? 1 : 2)))
 void decode_stream_kernel(
     DecodeKernelArgs a, const std::uint32_t* __restrict__ tables,
     const std::int32_t* __restrict__ lengths, float* __restrict__ out,
     float* __restrict__ part_o, float* __restrict__ part_ml, int* __restrict__ segments,
     const std::int64_t* __restrict__ append_slots) {
-  constexpr bool QLDS = stream_lds_query<PF, G>();
-  constexpr int S = QLDS ? kFp8StreamStage : kStreamStage;
+  constexpr int S = kStreamStage;
   __shared__ __align__(16) float s_p[2][8 * G];
   __shared__ __align__(16) float s_head[3][G];
   __shared__ __align__(16) float4 s_res_o[S][G][32];
@@ -1646,11 +1560,22 @@ void decode_stream_kernel(
   __shared__ __align__(16) float4 s_app_k[S][32];
   __shared__ __align__(16) float4 s_app_v[S][32];
   __shared__ long long s_app_dst[S];
-  __shared__ __align__(16) float4 s_qslot[QLDS ? 3 : 1][G][32];
-  decode_stream_body<G, APPEND, PF, false, S>(
+  decode_stream_body<G, APPEND, 0, false>(
       a, tables, lengths, out, part_o, part_ml, segments, append_slots, blockIdx.x, threadIdx.x,
-      StreamLds<G, S>{s_p, s_head, s_res_o, s_res_ml, s_res_dst, s_seg, s_seg_unit, s_app_k,
-                      s_app_v, s_app_dst, QLDS ? s_qslot : nullptr});
+      StreamLds<G>{s_p, s_head, s_res_o, s_res_ml, s_res_dst, s_seg, s_seg_unit, s_app_k,
+                   s_app_v, s_app_dst});
+}
+
+template <int G, bool APPEND, int PF>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(G == 8 ? 2 : mma_waves_per_simd(PF))))
+void decode_mma_kernel(
+    DecodeKernelArgs a, const std::uint32_t* __restrict__ tables,
+    const std::int32_t* __restrict__ lengths, float* __restrict__ out,
+    float* __restrict__ part_o, float* __restrict__ part_ml, int* __restrict__ segments,
+    const std::int64_t* __restrict__ append_slots) {
+  __shared__ __align__(1024) unsigned char lds[MmaGeom<G, PF>::kBytes];
+  decode_mma_body<G, APPEND, PF>(a, tables, lengths, out, part_o, part_ml, segments, append_slots,
+                                 static_cast<int>(blockIdx.x), static_cast<int>(threadIdx.x), lds);
 }
 
 // Cascade decode in one launch.  Blocks [0, prefix_blocks) are the cascade
@@ -2567,16 +2492,21 @@ namespace {
 
 
 // Wavefronts the stream kernel launches: every resident slot of the device
-// (fp32 and bf16 pages: two per SIMD up to four query heads per kv head, one
-// for eight; fp8 pages: four per SIMD up to four query heads, as the
-// kernels' register and LDS use allows), at most kMaxStreamWaves.
+// as the kernels' register and LDS use allows (fp32 pages: two per SIMD up to
+// four query heads per kv head, one for eight; bf16 and fp8 pages:
+// mma_waves_per_simd, two for eight query heads), at most kMaxStreamWaves.
 // beside_prefix: one per SIMD whatever the group, so the concurrent cascade
-// prefix pass finds registers on every SIMD.
-std::size_t stream_waves(std::size_t group, bool beside_prefix,
-                         PageType type = PageType::kF32) {
+// prefix pass finds registers on every SIMD.  compact: one for eight query
+// heads, because every wavefront takes a partial slot of the fixed scratch
+// that bounds the batch of the no-allocation entry.
+std::size_t stream_waves(std::size_t group, bool beside_prefix, PageType type, bool compact) {
   const int n = device_cus();
-  const std::size_t per_simd =
-      group >= 8 || beside_prefix ? 1 : (stream_lds_query_type(type) ? kFp8StreamWaves : 2);
+  std::size_t per_simd = 1;
+  if (!beside_prefix && group < 8) {
+    per_simd = type == PageType::kF32 ? 2 : mma_waves_per_simd(static_cast<int>(type));
+  } else if (!beside_prefix && type != PageType::kF32 && !compact) {
+    per_simd = 2;
+  }
   const std::size_t w = static_cast<std::size_t>(n) * 4 * per_simd;
   return w < kMaxStreamWaves ? w : kMaxStreamWaves;
 }
@@ -2587,9 +2517,15 @@ namespace {
 
 template <int G, bool APPEND, int PF>
 void launch_stream_variant(const dim3& grid, hipStream_t stream, const DecodeKernelArgs& k) {
-  decode_stream_kernel<G, APPEND, PF><<<grid, 64, 0, stream>>>(
-      k, k.tables, k.lengths, k.out, k.part_o, k.part_ml, k.segments,
-      APPEND ? k.append_slots : nullptr);
+  if constexpr (PF == 0) {
+    decode_stream_kernel<G, APPEND><<<grid, 64, 0, stream>>>(
+        k, k.tables, k.lengths, k.out, k.part_o, k.part_ml, k.segments,
+        APPEND ? k.append_slots : nullptr);
+  } else {
+    decode_mma_kernel<G, APPEND, PF><<<grid, 64, 0, stream>>>(
+        k, k.tables, k.lengths, k.out, k.part_o, k.part_ml, k.segments,
+        APPEND ? k.append_slots : nullptr);
+  }
 }
 
 template <int G, bool APPEND, int PF>
@@ -2666,6 +2602,7 @@ hipError_t launch_decode(const DecodeArgs& a, hipStream_t stream) {
   k.v_scale = a.page_type.v_scale;
   // fp8 keys widen to bare code values: their scale joins the score scale.
   if (a.page_type.type == PageType::kFP8) k.qscale *= a.page_type.k_scale;
+  k.rows_aligned = aligned16(a.query) && aligned16(a.tail_key) && aligned16(a.tail_value) ? 1 : 0;
   if (a.lengths == nullptr) return hipErrorInvalidValue;
   if (streamed) {
     // Cascade in one launch for groups up to kCascadeFusedMaxGroup (the
@@ -2675,7 +2612,7 @@ hipError_t launch_decode(const DecodeArgs& a, hipStream_t stream) {
     const bool fused = a.shared_pages > 0 && group <= kCascadeFusedMaxGroup;
     const bool overlap = !fused && a.shared_pages > 0 && a.side_stream != nullptr &&
                          a.fork_event != nullptr && a.join_event != nullptr;
-    const std::size_t waves = stream_waves(group, overlap || fused, a.page_type.type);
+    const std::size_t waves = stream_waves(group, overlap || fused, a.page_type.type, a.compact_layout);
     // The compact layout is sized for this launch's wavefront count (which
     // compact_decode_workspace_bytes gives for the same page type).
     if (a.compact_layout && a.shared_pages != 0) return hipErrorInvalidValue;
@@ -2818,7 +2755,7 @@ hipError_t launch_decode(const DecodeArgs& a, hipStream_t stream) {
 std::size_t compact_decode_workspace_bytes(std::size_t batch, std::size_t q_heads,
                                            std::size_t kv_heads, PageType type) {
   if (kv_heads == 0 || q_heads % kv_heads != 0) return 0;
-  return stream_layout(batch, q_heads, kv_heads, stream_waves(q_heads / kv_heads, false, type), 0)
+  return stream_layout(batch, q_heads, kv_heads, stream_waves(q_heads / kv_heads, false, type, true), 0)
       .total;
 }
 
