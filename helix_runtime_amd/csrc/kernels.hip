@@ -1616,43 +1616,45 @@ void cascade_decode_kernel(
       stream_lds(sh.stream[w]));
 }
 
-// Combines the partials of units that span several stream wavefronts.  One
-// workgroup of G * 32 threads per unit (kv head major: unit = kvh * batch +
-// b); thread (h, d4) owns 4 output dims of query head h.  The unit's
-// wavefront range was recorded by the stream kernel, so the partial loads
-// are issued at once.
-template <int G>
-__global__ __launch_bounds__(256) void decode_stream_merge_kernel(DecodeKernelArgs a) {
+// Combines the partials of units that span several stream wavefronts.  A
+// workgroup takes HB query heads of one unit (kv head major: kvh * batch +
+// b): per head, group g of NG groups of 32 threads takes the unit's partials
+// g, g + NG, ... with L of them loaded at once, thread d4 of a group 4
+// output dims; the groups' results are combined through LDS.
+template <int G, int NG, int HB, int L>
+__global__ __launch_bounds__(HB * NG * 32) void decode_stream_merge_kernel(DecodeKernelArgs a) {
   constexpr int D = 128;
-  const int unit = blockIdx.x;
+  constexpr int kBlocks = G / HB;  // workgroups per unit
+  __shared__ __align__(16) float4 s_o[HB][NG][32];
+  __shared__ float s_ml[HB][NG][2];
+  const int unit = static_cast<int>(blockIdx.x) / kBlocks;
+  const int hb = static_cast<int>(threadIdx.x) / (NG * 32);
+  const int h = static_cast<int>(blockIdx.x) % kBlocks * HB + hb;
   const int2 seg = reinterpret_cast<const int2*>(a.segments)[unit];
   const bool cascade = a.first_page > 0;
   if (seg.y <= 1 && !cascade) return;
   const int kvh = unit / a.batch;
   const int b = unit % a.batch;
-  const int tid = threadIdx.x;
-  const int h = tid / (D / 4);
-  const int d4 = tid % (D / 4);
+  const int grp = static_cast<int>(threadIdx.x) / 32 % NG;
+  const int d4 = static_cast<int>(threadIdx.x) % 32;
   const std::size_t slot0 = static_cast<std::size_t>(unit) + seg.x;
-  // Online merge over chunks of 8 partials; each chunk's loads issue together.
-  constexpr int kChunk = 8;
   float mx = -INFINITY;
   float den = 0.0f;
   float4 num = make_float4(0.f, 0.f, 0.f, 0.f);
   // Partials: the unit's stream segments, then (cascade) its prefix chunks.
   const int nparts = seg.y + (cascade ? a.prefix_chunks : 0);
   const long long units = static_cast<long long>(a.batch) * a.kv_heads;
-  for (int s0 = 0; s0 < nparts; s0 += kChunk) {
-    float ms[kChunk], ls[kChunk];
-    float4 os[kChunk];
+  for (int s0 = grp; s0 < nparts; s0 += NG * L) {
+    float ms[L], ls[L];
+    float4 os[L];
 #pragma unroll
-    for (int i = 0; i < kChunk; ++i) {
-      const bool in = s0 + i < nparts;
+    for (int i = 0; i < L; ++i) {
+      const int s = s0 + i * NG;
+      const bool in = s < nparts;
       const std::size_t slot =
           !in ? slot0
-              : (s0 + i < seg.y
-                     ? slot0 + s0 + i
-                     : static_cast<std::size_t>(a.prefix_slot0 + (s0 + i - seg.y) * units + unit));
+              : (s < seg.y ? slot0 + s
+                           : static_cast<std::size_t>(a.prefix_slot0 + (s - seg.y) * units + unit));
       ms[i] = in ? a.part_ml[(slot * G + h) * 2] : -INFINITY;
       ls[i] = in ? a.part_ml[(slot * G + h) * 2 + 1] : 0.0f;
       os[i] = in ? reinterpret_cast<const float4*>(a.part_o + (slot * G + h) * D)[d4]
@@ -1660,7 +1662,7 @@ __global__ __launch_bounds__(256) void decode_stream_merge_kernel(DecodeKernelAr
     }
     float cm = mx;
 #pragma unroll
-    for (int i = 0; i < kChunk; ++i) cm = fmaxf(cm, ms[i]);
+    for (int i = 0; i < L; ++i) cm = fmaxf(cm, ms[i]);
     const float sc = exp2_ratio(mx, cm);
     den *= sc;
     num.x *= sc;
@@ -1668,8 +1670,8 @@ __global__ __launch_bounds__(256) void decode_stream_merge_kernel(DecodeKernelAr
     num.z *= sc;
     num.w *= sc;
 #pragma unroll
-    for (int i = 0; i < kChunk; ++i) {
-      const float w = s0 + i < nparts ? exp2_ratio(ms[i], cm) : 0.0f;
+    for (int i = 0; i < L; ++i) {
+      const float w = s0 + i * NG < nparts ? exp2_ratio(ms[i], cm) : 0.0f;
       den += w * ls[i];
       num.x += w * os[i].x;
       num.y += w * os[i].y;
@@ -1677,6 +1679,28 @@ __global__ __launch_bounds__(256) void decode_stream_merge_kernel(DecodeKernelAr
       num.w += w * os[i].w;
     }
     mx = cm;
+  }
+  if constexpr (NG > 1) {
+    s_o[hb][grp][d4] = num;
+    if (d4 == 0) {
+      s_ml[hb][grp][0] = mx;
+      s_ml[hb][grp][1] = den;
+    }
+    __syncthreads();
+    if (grp != 0) return;
+    const int live = nparts < NG ? nparts : NG;
+    for (int g = 1; g < live; ++g) mx = fmaxf(mx, s_ml[hb][g][0]);
+    den = 0.0f;
+    num = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int g = 0; g < live; ++g) {
+      const float w = exp2_ratio(s_ml[hb][g][0], mx);
+      const float4 o = s_o[hb][g][d4];
+      den += w * s_ml[hb][g][1];
+      num.x += w * o.x;
+      num.y += w * o.y;
+      num.z += w * o.z;
+      num.w += w * o.w;
+    }
   }
   float4 r;
   if (mx == -INFINITY) {
@@ -2573,6 +2597,43 @@ void launch_stream(const dim3& grid, hipStream_t stream, const DecodeKernelArgs&
   });
 }
 
+// The merge is bound by latency: a unit has about as many partials as the
+// launch has wavefronts over units, from a handful in a full batch to
+// hundreds for one long sequence, and one group reading those 8 at a time
+// took longer than the attention.  More groups per row cut that chain, as
+// long as the launch stays around what the CUs hold at once (2048 threads
+// each).  One layer with its merge, us, 32/8 heads unless said: one sequence
+// of 4000 tokens, fp32 65 -> 23 and fp8 58 -> 17 (27 and 21 with 8 groups);
+// 4 of 100-2000, fp32 37 -> 20; 8 x 32 heads of 128-2048 tokens (1 head per
+// row group) 40.1 -> 38.2 (8 groups; 38.4 with 4); 64 sequences, fp32 225.3
+// -> 224.3 (4 groups; 225.4 with 8); 128 forks of one prompt 62.9 with one
+// group, 64.7 with 4, 66.4 with 8.
+template <int G>
+void launch_stream_merge_group(hipStream_t stream, const DecodeKernelArgs& k) {
+  const unsigned units = static_cast<unsigned>(k.batch) * static_cast<unsigned>(k.kv_heads);
+  const unsigned rows = units * G;
+  if (rows >= 4096) {
+    decode_stream_merge_kernel<G, 1, G, 8><<<units, G * 32, 0, stream>>>(k);
+  } else if (rows >= 2048) {
+    decode_stream_merge_kernel<G, 4, 1, 4><<<rows, 128, 0, stream>>>(k);
+  } else if (rows >= 512) {
+    decode_stream_merge_kernel<G, 8, 1, 4><<<rows, 256, 0, stream>>>(k);
+  } else {
+    decode_stream_merge_kernel<G, 16, 1, 4><<<rows, 512, 0, stream>>>(k);
+  }
+}
+
+hipError_t launch_stream_merge(std::size_t group, hipStream_t stream, const DecodeKernelArgs& k) {
+  switch (group) {
+    case 1: launch_stream_merge_group<1>(stream, k); break;
+    case 2: launch_stream_merge_group<2>(stream, k); break;
+    case 4: launch_stream_merge_group<4>(stream, k); break;
+    case 8: launch_stream_merge_group<8>(stream, k); break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
 }  // namespace
 
 hipError_t launch_decode(const DecodeArgs& a, hipStream_t stream) {
@@ -2664,14 +2725,7 @@ hipError_t launch_decode(const DecodeArgs& a, hipStream_t stream) {
           e = hipEventRecord(a.between_event, stream);
           if (e != hipSuccess) return e;
         }
-        const dim3 mgrid(static_cast<unsigned>(a.batch * a.kv_heads));
-        switch (group) {
-          case 1: decode_stream_merge_kernel<1><<<mgrid, 1 * 32, 0, stream>>>(k); break;
-          case 2: decode_stream_merge_kernel<2><<<mgrid, 2 * 32, 0, stream>>>(k); break;
-          case 4: decode_stream_merge_kernel<4><<<mgrid, 4 * 32, 0, stream>>>(k); break;
-          default: return hipErrorInvalidValue;
-        }
-        return hipGetLastError();
+        return launch_stream_merge(group, stream, k);
       }
       if (overlap) {
         hipError_t e = hipEventRecord(a.fork_event, stream);
@@ -2713,15 +2767,7 @@ hipError_t launch_decode(const DecodeArgs& a, hipStream_t stream) {
       e = hipStreamWaitEvent(stream, a.join_event, 0);
       if (e != hipSuccess) return e;
     }
-    const dim3 mgrid(static_cast<unsigned>(a.batch * a.kv_heads));
-    switch (group) {
-      case 1: decode_stream_merge_kernel<1><<<mgrid, 1 * 32, 0, stream>>>(k); break;
-      case 2: decode_stream_merge_kernel<2><<<mgrid, 2 * 32, 0, stream>>>(k); break;
-      case 4: decode_stream_merge_kernel<4><<<mgrid, 4 * 32, 0, stream>>>(k); break;
-      case 8: decode_stream_merge_kernel<8><<<mgrid, 8 * 32, 0, stream>>>(k); break;
-      default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
+    return launch_stream_merge(group, stream, k);
   }
   const WorkspaceLayout lay = layout_for(a.batch, a.q_heads, a.kv_heads, max_splits);
   k.part_o = reinterpret_cast<float*>(ws + lay.part_o);
