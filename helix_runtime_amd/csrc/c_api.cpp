@@ -513,7 +513,8 @@ void run_reference_attention(const AttentionShape& s, const float* query,
                              const float* key_blocks, const float* value_blocks,
                              const std::uint32_t* block_table, const float* tail_key,
                              const float* tail_value, float* output, float* workspace,
-                             std::size_t workspace_elements, hipStream_t stream, const char* op) {
+                             std::size_t workspace_elements, bool scalar, hipStream_t stream,
+                             const char* op) {
   if (!validate_reference_buffers(s, query, key_blocks, value_blocks, block_table, tail_key,
                                   tail_value, output, workspace, workspace_elements, op)) {
     return;
@@ -537,7 +538,12 @@ void run_reference_attention(const AttentionShape& s, const float* query,
   a.history = s.history;
   a.tail = s.tail;
   a.offset = s.offset;
-  helix::hip_check(helix::hip::launch_generic(a, stream), (std::string(op) + " launch").c_str());
+  // The scalar kernel keeps the probability entry (the reference's loop
+  // order) and head sizes past the matrix-core kernel's.
+  const hipError_t e = !scalar && helix::hip::tiled_attention_fits(a)
+                           ? helix::hip::launch_tiled_attention(a, stream)
+                           : helix::hip::launch_generic(a, stream);
+  helix::hip_check(e, (std::string(op) + " launch").c_str());
 }
 
 // Device scratch of the reference-shaped fast routes, one buffer per
@@ -743,7 +749,7 @@ int helix_paged_attention_out(const float* query, size_t q_heads, size_t queries
       return;
     }
     run_reference_attention(s, query, key_blocks, value_blocks, block_table, nullptr, nullptr,
-                            output, score_workspace, workspace_elements, as_stream(stream), op);
+                            output, score_workspace, workspace_elements, false, as_stream(stream), op);
   });
 }
 
@@ -778,7 +784,8 @@ void attention_with_tail(const float* query, size_t q_heads, size_t tail_tokens,
     }
   }
   run_reference_attention(s, query, key_blocks, value_blocks, block_table, tail_key, tail_value,
-                          output, score_workspace, workspace_elements, as_stream(stream), op);
+                          output, score_workspace, workspace_elements, probabilities,
+                          as_stream(stream), op);
 }
 
 }  // namespace

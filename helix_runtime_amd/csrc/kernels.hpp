@@ -253,6 +253,12 @@ struct GenericArgs {
 
 hipError_t launch_generic(const GenericArgs& a, hipStream_t stream);
 
+// The same call on the fp32 matrix cores (tiled_attention.hip): head sizes
+// up to 256 and 32-bit key and row counts (tiled_attention_fits).  Softmax
+// rules and workspace contract as above; sums in another order.
+bool tiled_attention_fits(const GenericArgs& a);
+hipError_t launch_tiled_attention(const GenericArgs& a, hipStream_t stream);
+
 // ------------------------------------------------------- chunked prefill ----
 // Batched chunked-prefill attention (MFMA): every sequence b attends with
 // `tokens` query rows to its paged history (lengths[b] tokens through row b
