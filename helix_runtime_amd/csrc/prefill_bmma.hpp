@@ -34,10 +34,16 @@
 // is key 4 g + j for j < 4 and key 16 + 4 g + j - 4 otherwise, and V is
 // staged in the same order.
 //
-// LDS: K rows as bf16, padded to kBKStride elements (16 bytes) so the 16
-// rows one operand read touches start in distinct banks; V transposed,
-// [dim][contraction index] with rows of kVtStride elements, so one 16-byte
-// read gives a lane the 8 keys of one dim that the P.V operand needs.
+// LDS: K and V rows as bf16 in key order, 256 bytes a row, their 16-byte
+// chunks XOR-swizzled by row.  V is transposed on the way out
+// (ds_read_b64_tr_b16: the 4 keys of one dim that a lane's score tile left
+// it), so staging writes rows and bf16 pages need no staging code at all:
+// they go from global memory to LDS directly.  Storing V transposed instead
+// took four 2-byte LDS stores a thread and page, and every page went through
+// registers.  16 sequences of 512 rows over 0-4096 tokens, 32/8 heads: bf16
+// pages 965 -> 750 us, fp8 pages 1013 -> 805 us (their codes are widened
+// once per workgroup on the way; widening them in the operand reads would
+// repeat it in all eight wavefronts).
 #pragma once
 
 #include "prefill_body.hpp"
@@ -47,22 +53,34 @@ namespace helix::hip::prefill_detail {
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef short v8s __attribute__((ext_vector_type(8)));
 
-constexpr int kBKeys = 2 * P;          // keys per LDS stage
-constexpr int kBKStride = D + 8;       // bf16 elements per K row in LDS
-constexpr int kVtStride = kBKeys + 8;  // bf16 elements per transposed V row
+typedef short v4s __attribute__((ext_vector_type(4)));
+
+constexpr int kBKeys = 2 * P;  // keys per LDS stage
 
 struct PrefillBmmaShared {
-  __align__(16) unsigned short k[2][kBKeys * kBKStride];
-  __align__(16) unsigned short vt[2][D * kVtStride];
+  __align__(1024) unsigned short k[2][kBKeys * D];
+  __align__(1024) unsigned short v[2][kBKeys * D];
   // The low bf16 term of each lane's query operand, [wave][step][lane]:
   // kept here rather than in registers, which the other two terms, the
   // accumulators and the staging fill.
   __align__(16) uint4 qlo[kRows / 16][4][64];
 };
 
-// Position of key kr (0 .. 31 within a stage) on the P.V contraction axis.
-__device__ __forceinline__ int bmma_key_slot(int kr) {
-  return 8 * ((kr & 15) >> 2) + 4 * (kr >> 4) + (kr & 3);
+// Byte position in a stage of 16-byte chunk `chunk` of row `row` (keys 0 ..
+// 31): chunks are XOR-swizzled by row, so that the operand reads (K: one
+// chunk of 16 rows; V: one pair of chunks of 8 rows) hit distinct banks.
+__device__ __forceinline__ unsigned bmma_k_at(int row, int chunk) {
+  return static_cast<unsigned>(row * (2 * D) + ((chunk ^ row) & 15) * 16);
+}
+__device__ __forceinline__ unsigned bmma_v_at(int row, int chunk) {
+  return static_cast<unsigned>(row * (2 * D) + (chunk ^ (2 * (row & 7))) * 16);
+}
+
+// A uniform read of memory that the kernel does not write, through the
+// scalar cache.
+__device__ __forceinline__ std::uint32_t uniform_read(const std::uint32_t* p) {
+  return *(const __attribute__((address_space(4))) std::uint32_t*)(
+      reinterpret_cast<std::uintptr_t>(p));
 }
 
 // x = hi + mid + lo exactly (truncating splits of a finite fp32); a
@@ -125,7 +143,6 @@ __device__ __forceinline__ void prefill_body_bmma(PrefillKernelArgs a,
                                                   std::uint32_t* __restrict__ redo,
                                                   std::uint32_t block, PrefillBmmaShared& sh) {
   static_assert(PF == 1 || PF == 2, "bf16 matrix-core prefill is for bf16 and fp8 pages");
-  constexpr int RP = 16 / RT;  // key rows per staging pass
   constexpr int PW = kRows / G;
   constexpr bool FP8 = PF == 2;
 
@@ -148,7 +165,7 @@ __device__ __forceinline__ void prefill_body_bmma(PrefillKernelArgs a,
   const int T = a.tokens;
   const int pos0 = pb * PW;
 
-  int hist = a.lengths[b];
+  int hist = __builtin_amdgcn_readfirstlane(a.lengths[b]);
   bool bad = hist < 0 || hist > a.max_blocks * P;
   if (bad) hist = 0;
   const int key_end = hist + min(T, pos0 + PW);
@@ -202,105 +219,169 @@ __device__ __forceinline__ void prefill_body_bmma(PrefillKernelArgs a,
     l[t] = 0.f;
   }
 
-  // Staging: thread tid moves dims 4 scol .. + 3 of key rows srow + RP r
-  // (r < NR) of one 16-key half (one page) of a 32-key block, for K and V
-  // (as loaded: bf16 words, fp8 code words or fp32 chunk rows).  The two
-  // halves of the next block are staged one after the other, so only one
-  // page is held in registers.
-  constexpr int NR = P / RP;
+  // Staging of a 16-key half (one page) of the next 32-key block.
+  // - A bf16 page wholly in the history goes straight from global memory to
+  //   LDS as stored: 4 wavefronts per half, each 1 KiB (4 rows) of the K page
+  //   and of the V page.
+  // - Everything else goes through registers: fp8 codes (widened on the way),
+  //   chunk rows (rounded onto the page grid), zeros past the key range.
+  //   Thread tid moves dims 4 scol .. + 3 of key row srow, the two halves one
+  //   after the other, so only one page is held in registers.  The one bf16
+  //   half where the history ends inside a page is loaded when it is stored,
+  //   so that the loads of the others are of one kind (chunk rows).
+  static_assert(RT == 1, "eight wavefronts stage a block");
   const int srow = tid >> 5;
   const int scol = tid & 31;
-  float4 stk[NR], stv[NR];
+  const int uwave = __builtin_amdgcn_readfirstlane(wave);
+  auto direct = [&](int blk, int half) { return !FP8 && blk * kBKeys + half * P + P <= hist; };
+  auto chunk_only = [&](int blk, int half) { return blk * kBKeys + half * P >= hist; };
+  const int drow = 4 * (uwave & 3) + grp;  // row within the page
+  const unsigned dk = bmma_k_at(drow, col), dv = bmma_v_at(drow, col);  // chunk at position col
+  // Physical page of this wavefront's half of block blk (read a block ahead
+  // of its loads).
+  auto direct_page = [&](int blk) -> std::uint32_t {
+    const int half = uwave >> 2;
+    return direct(blk, half) ? uniform_read(table + blk * 2 + half) : 0u;
+  };
+  auto direct_load = [&](int buf, int blk, std::uint32_t page) {
+    const int half = uwave >> 2;
+    if (!direct(blk, half)) return;
+    const unsigned at = static_cast<unsigned>(half * P * 2 * D + (uwave & 3) * 1024);
+    // A page outside the pool is not read: zeros in its place.
+    const bool ok = page < a.physical_blocks;
+    bad = bad || !ok;
+    const std::size_t off = (static_cast<std::size_t>(page) * a.kv_heads + kvh) * (P * D * 2);
+    const auto* kb = ok ? reinterpret_cast<const unsigned char*>(a.key_pool) + off
+                        : reinterpret_cast<const unsigned char*>(kZeroRows);
+    const auto* vb = ok ? reinterpret_cast<const unsigned char*>(a.value_pool) + off
+                        : reinterpret_cast<const unsigned char*>(kZeroRows);
+    lds_load16_at(kb, ok ? dk : lane * 16u,
+                  lds_address(reinterpret_cast<unsigned char*>(sh.k[buf]) + at));
+    lds_load16_at(vb, ok ? dv : lane * 16u,
+                  lds_address(reinterpret_cast<unsigned char*>(sh.v[buf]) + at));
+  };
+  const float* const chunk_k = a.chunk_key + chunk_row0 * D;
+  const float* const chunk_v = a.chunk_value + chunk_row0 * D;
+  float4 stk = make_float4(0.f, 0.f, 0.f, 0.f), stv = stk;
   auto stage_load = [&](int blk, int half) {
     const int pkey0 = blk * kBKeys + half * P;
-    std::size_t page_off = 0;
-    bool page_ok = false;
-    if (pkey0 < hist) {
-      const std::uint32_t page = table[pkey0 / P];
-      page_ok = page < a.physical_blocks;
-      bad = bad || !page_ok;
-      page_off = page_ok ? (static_cast<std::size_t>(page) * a.kv_heads + kvh) * P * D : 0;
-    }
-#pragma unroll
-    for (int r = 0; r < NR; ++r) {
-      const int key = pkey0 + srow + RP * r;
+    if constexpr (FP8) {
+      const int key = pkey0 + srow;
       const bool in_hist = key < hist;
-      const bool valid = key < key_end && (!in_hist || page_ok);
-      const int off = (srow + RP * r) * D + scol * 4;
-      stk[r] = make_float4(0.f, 0.f, 0.f, 0.f);
-      stv[r] = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (valid && in_hist) {
-        const std::size_t e = page_off + off;
-        if constexpr (FP8) {
-          stk[r].x = __uint_as_float(*reinterpret_cast<const unsigned*>(
-              reinterpret_cast<const unsigned char*>(a.key_pool) + e));
-          stv[r].x = __uint_as_float(*reinterpret_cast<const unsigned*>(
-              reinterpret_cast<const unsigned char*>(a.value_pool) + e));
-        } else {
-          const uint2 kw = *reinterpret_cast<const uint2*>(
-              reinterpret_cast<const unsigned short*>(a.key_pool) + e);
-          const uint2 vw = *reinterpret_cast<const uint2*>(
-              reinterpret_cast<const unsigned short*>(a.value_pool) + e);
-          stk[r] = make_float4(__uint_as_float(kw.x), __uint_as_float(kw.y), 0.f, 0.f);
-          stv[r] = make_float4(__uint_as_float(vw.x), __uint_as_float(vw.y), 0.f, 0.f);
-        }
-      } else if (valid) {
-        const std::size_t crow = chunk_row0 + static_cast<std::size_t>(key - hist);
-        stk[r] = *reinterpret_cast<const float4*>(a.chunk_key + crow * D + scol * 4);
-        stv[r] = *reinterpret_cast<const float4*>(a.chunk_value + crow * D + scol * 4);
+      std::size_t page_off = 0;
+      bool page_ok = false;
+      if (pkey0 < hist) {
+        const std::uint32_t page = uniform_read(table + pkey0 / P);
+        page_ok = page < a.physical_blocks;
+        bad = bad || !page_ok;
+        page_off = page_ok ? (static_cast<std::size_t>(page) * a.kv_heads + kvh) * P * D : 0;
       }
+      stk = stv = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (in_hist) {
+        if (page_ok) {  // the row's 4 codes in .x
+          const std::size_t e = page_off + srow * D + scol * 4;
+          stk.x = __uint_as_float(*reinterpret_cast<const unsigned*>(
+              reinterpret_cast<const unsigned char*>(a.key_pool) + e));
+          stv.x = __uint_as_float(*reinterpret_cast<const unsigned*>(
+              reinterpret_cast<const unsigned char*>(a.value_pool) + e));
+        }
+      } else if (key < key_end) {
+        const unsigned at = static_cast<unsigned>((key - hist) * D + scol * 4);
+        stk = *reinterpret_cast<const float4*>(chunk_k + at);
+        stv = *reinterpret_cast<const float4*>(chunk_v + at);
+      }
+    } else if (chunk_only(blk, half)) {
+      // (A chunk's rows fit 32-bit offsets: 2^25 rows of one head are 16 GB.)
+      const unsigned at =
+          static_cast<unsigned>((min(pkey0 + srow, key_end - 1) - hist) * D + scol * 4);
+      stk = *reinterpret_cast<const float4*>(chunk_k + at);
+      stv = *reinterpret_cast<const float4*>(chunk_v + at);
     }
   };
-  // Stores a staged half as bf16 (K rows, V transposed in contraction order).
+  // Stores a staged half as bf16 rows (fp8: the bare code values).
   auto stage_store = [&](int buf, int blk, int half) {
-#pragma unroll
-    for (int r = 0; r < NR; ++r) {
-      const int kr = half * P + srow + RP * r;
-      const int key = blk * kBKeys + kr;
-      uint2 kb, vb;  // 4 bf16 each, low half first (fp8: the bare code values)
-      if (key < hist) {
-        if constexpr (FP8) {
-          kb = fp8_codes_bf16(__float_as_uint(stk[r].x));
-          vb = fp8_codes_bf16(__float_as_uint(stv[r].x));
-        } else {
-          kb = make_uint2(__float_as_uint(stk[r].x), __float_as_uint(stk[r].y));
-          vb = make_uint2(__float_as_uint(stv[r].x), __float_as_uint(stv[r].y));
-        }
+    if (direct(blk, half)) return;
+    const int kr = half * P + srow;
+    const int key = blk * kBKeys + kr;
+    uint2 kb, vb;  // 4 bf16 each, low half first
+    auto rounded = [&](const float4& k, const float4& v) {
+      if constexpr (FP8) {
+        kb = fp8_codes_bf16(fp8_pack4_scaled(k, a.k_scale));
+        vb = fp8_codes_bf16(fp8_pack4_scaled(v, a.v_scale));
       } else {
-        // Chunk rows (zeros past the key range): onto the page grid.
-        if constexpr (FP8) {
-          kb = fp8_codes_bf16(fp8_pack4_scaled(stk[r], a.k_scale));
-          vb = fp8_codes_bf16(fp8_pack4_scaled(stv[r], a.v_scale));
-        } else {
-          kb = make_uint2(bf16_pack(stk[r].x, stk[r].y), bf16_pack(stk[r].z, stk[r].w));
-          vb = make_uint2(bf16_pack(stv[r].x, stv[r].y), bf16_pack(stv[r].z, stv[r].w));
-        }
+        kb = make_uint2(bf16_pack(k.x, k.y), bf16_pack(k.z, k.w));
+        vb = make_uint2(bf16_pack(v.x, v.y), bf16_pack(v.z, v.w));
       }
-      *reinterpret_cast<uint2*>(&sh.k[buf][kr * kBKStride + scol * 4]) = kb;
-      unsigned short* vt = &sh.vt[buf][(scol * 4) * kVtStride + bmma_key_slot(kr)];
-      vt[0] = static_cast<unsigned short>(vb.x & 0xffffu);
-      vt[kVtStride] = static_cast<unsigned short>(vb.x >> 16);
-      vt[2 * kVtStride] = static_cast<unsigned short>(vb.y & 0xffffu);
-      vt[3 * kVtStride] = static_cast<unsigned short>(vb.y >> 16);
+    };
+    if constexpr (FP8) {
+      if (key < hist) {
+        kb = fp8_codes_bf16(__float_as_uint(stk.x));
+        vb = fp8_codes_bf16(__float_as_uint(stv.x));
+      } else {
+        rounded(stk, stv);
+      }
+    } else if (chunk_only(blk, half)) {
+      rounded(stk, stv);
+      if (key >= key_end) kb = vb = make_uint2(0u, 0u);
+    } else {
+      const int pkey0 = blk * kBKeys + half * P;
+      const std::uint32_t page = uniform_read(table + pkey0 / P);
+      const bool ok = page < a.physical_blocks;
+      bad = bad || !ok;
+      kb = vb = make_uint2(0u, 0u);
+      if (key < hist) {
+        if (ok) {
+          const std::size_t e =
+              (static_cast<std::size_t>(page) * a.kv_heads + kvh) * P * D + srow * D + scol * 4;
+          kb = *reinterpret_cast<const uint2*>(
+              reinterpret_cast<const unsigned short*>(a.key_pool) + e);
+          vb = *reinterpret_cast<const uint2*>(
+              reinterpret_cast<const unsigned short*>(a.value_pool) + e);
+        }
+      } else if (key < key_end) {
+        const unsigned at = static_cast<unsigned>((key - hist) * D + scol * 4);
+        rounded(*reinterpret_cast<const float4*>(chunk_k + at),
+                *reinterpret_cast<const float4*>(chunk_v + at));
+      }
     }
+    const unsigned part = static_cast<unsigned>((scol & 1) * 8);
+    *reinterpret_cast<uint2*>(reinterpret_cast<unsigned char*>(sh.k[buf]) +
+                              bmma_k_at(kr, scol >> 1) + part) = kb;
+    *reinterpret_cast<uint2*>(reinterpret_cast<unsigned char*>(sh.v[buf]) +
+                              bmma_v_at(kr, scol >> 1) + part) = vb;
   };
 
   __shared__ int s_redo;
   if (tid == 0) s_redo = 0;  // published by the first barrier below
   const int nblocks = (key_end + kBKeys - 1) / kBKeys;
+  auto block_barrier = [&]() {
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  };
+  std::uint32_t page_ahead = 0;
   if (nblocks > 0) {
+    direct_load(0, 0, direct_page(0));
+    page_ahead = direct_page(1);
     stage_load(0, 0);
     stage_store(0, 0, 0);
     stage_load(0, 1);
     stage_store(0, 0, 1);
   }
-  __syncthreads();
+  block_barrier();
+  // Operand reads: K row 16 h + col, chunk 4 s + grp; V rows 4 grp .. + 3 of
+  // a page, 16 dims of tile dt, transposed on the way out of LDS.
+  const unsigned kop_at = bmma_k_at(col, grp);
+  const int vrow = 4 * grp + (col >> 2);
+  const unsigned vop_at = bmma_v_at(vrow, 0) + static_cast<unsigned>((col & 3) * 8);
   for (int n = 0; n < nblocks; ++n) {
     const int buf = n & 1;
     const bool next = n + 1 < nblocks;
-    if (next) stage_load(n + 1, 0);
-    const unsigned short* K = sh.k[buf];
-    const unsigned short* VT = sh.vt[buf];
+    if (next) {
+      direct_load(buf ^ 1, n + 1, page_ahead);
+      page_ahead = direct_page(n + 2);
+      stage_load(n + 1, 0);
+    }
+    const unsigned char* K = reinterpret_cast<const unsigned char*>(sh.k[buf]);
+    const unsigned char* V = reinterpret_cast<const unsigned char*>(sh.v[buf]);
 
     // S^T = K Q^T on the bf16 matrix cores: st[t][h] holds keys
     // 16 h + 4 grp + i of query row t * 16 + col.
@@ -319,8 +400,7 @@ __device__ __forceinline__ void prefill_body_bmma(PrefillKernelArgs a,
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           const v8bf kop = __builtin_bit_cast(
-              v8bf,
-              *reinterpret_cast<const v8s*>(&K[(16 * h + col) * kBKStride + 32 * s + 8 * grp]));
+              v8bf, *reinterpret_cast<const v8s*>(K + h * (P * 2 * D) + (kop_at ^ (64u * s))));
           st[t][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kop, qlo, st[t][h], 0, 0, 0);
 #pragma unroll
           for (int term = 1; term >= 0; --term) {
@@ -359,9 +439,9 @@ __device__ __forceinline__ void prefill_body_bmma(PrefillKernelArgs a,
 #pragma unroll
           for (int j = 0; j < 8; ++j) p[t][j] = vis[j] ? exp2_ratio(x[j], mn) : 0.f;
         }
-        const float sum = row_sum(((p[t][0] + p[t][1]) + (p[t][2] + p[t][3])) +
-                                  ((p[t][4] + p[t][5]) + (p[t][6] + p[t][7])));
-        l[t] = l[t] * alpha + sum;
+        // The lane's own keys; the row's four lanes are added at the end.
+        l[t] = l[t] * alpha + (((p[t][0] + p[t][1]) + (p[t][2] + p[t][3])) +
+                               ((p[t][4] + p[t][5]) + (p[t][6] + p[t][7])));
         m[t] = mn;
       }
     };
@@ -395,8 +475,12 @@ __device__ __forceinline__ void prefill_body_bmma(PrefillKernelArgs a,
       __builtin_amdgcn_s_setprio(1);
 #pragma unroll
       for (int dt = 0; dt < 8; ++dt) {
+        using LdsV4s = __attribute__((address_space(3))) v4s;
+        const unsigned char* vp = V + (vop_at ^ (32u * dt));
+        const v4s v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsV4s*)(vp));
+        const v4s v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsV4s*)(vp + P * 2 * D));
         const v8bf vop = __builtin_bit_cast(
-            v8bf, *reinterpret_cast<const v8s*>(&VT[(16 * dt + col) * kVtStride + 8 * grp]));
+            v8bf, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
 #pragma unroll
         for (int t = 0; t < RT; ++t) {
 #pragma unroll
@@ -410,12 +494,13 @@ __device__ __forceinline__ void prefill_body_bmma(PrefillKernelArgs a,
 
     __builtin_amdgcn_s_setprio(0);
     if (next) stage_store(buf ^ 1, n + 1, 1);
-    __syncthreads();
+    block_barrier();
   }
 
   bool nan_row = false;
 #pragma unroll
   for (int t = 0; t < RT; ++t) {
+    l[t] = row_sum(l[t]);
     nan_row = nan_row || !(l[t] < INFINITY);  // NaN, or a sum that overflowed
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt)

@@ -200,6 +200,14 @@ __device__ __forceinline__ void lds_load16(const void* src, unsigned lds) {
   asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "{m0}"(lds) : "memory");
 }
 
+// The same from a uniform base and a byte offset per lane.
+__device__ __forceinline__ void lds_load16_at(const void* base, unsigned off, unsigned lds) {
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+               :
+               : "v"(off), "s"(base), "{m0}"(lds)
+               : "memory");
+}
+
 __device__ __forceinline__ unsigned lds_address(const void* p) {
   return __builtin_amdgcn_readfirstlane(
       static_cast<unsigned>(reinterpret_cast<std::uintptr_t>(p)));
