@@ -2607,12 +2607,15 @@ void launch_stream(const dim3& grid, hipStream_t stream, const DecodeKernelArgs&
 // 4 of 100-2000, fp32 37 -> 20; 8 x 32 heads of 128-2048 tokens (1 head per
 // row group) 40.1 -> 38.2 (8 groups; 38.4 with 4); 64 sequences, fp32 225.3
 // -> 224.3 (4 groups; 225.4 with 8); 128 forks of one prompt 62.9 with one
-// group, 64.7 with 4, 66.4 with 8.
+// group, 64.7 with 4, 66.4 with 8; 22 of 98 tokens (8 partials each), fp32
+// 15.7 with one group, 16.1 with 8.
 template <int G>
 void launch_stream_merge_group(hipStream_t stream, const DecodeKernelArgs& k) {
   const unsigned units = static_cast<unsigned>(k.batch) * static_cast<unsigned>(k.kv_heads);
   const unsigned rows = units * G;
-  if (rows >= 4096) {
+  // No unit has more partials than pages: up to 8 are read at once anyway.
+  const bool few = k.max_blocks - k.first_page + 1 + k.prefix_chunks <= 8;
+  if (few || rows >= 4096) {
     decode_stream_merge_kernel<G, 1, G, 8><<<units, G * 32, 0, stream>>>(k);
   } else if (rows >= 2048) {
     decode_stream_merge_kernel<G, 4, 1, 4><<<rows, 128, 0, stream>>>(k);
