@@ -1282,7 +1282,8 @@ def main():
         "decode_merge_avg_us": round(float(np.mean(merge_ms)) * 1e3, 2),
         "decode_kernel": ("decode_split_kernel" if split != 0 else
                           "cascade_decode_kernel" if batch.shared_pages() > 0 else
-                          "decode_stream_kernel"),
+                          "decode_stream_kernel" if args.page_dtype == "f32" else
+                          "decode_mma_kernel"),
         "roofline": {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBPS,
                      "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBPS, 4),
                      "traffic": traffic},

@@ -31,8 +31,8 @@
 // 4 g + i and 16 + 4 g + i of row col in lane (g = lane / 16, col = lane %
 // 16).  P.V contracts over the keys in any order, so its 32-key operand
 // takes them in the order the scores left them: contraction index 8 g + j
-// is key 4 g + j for j < 4 and key 16 + 4 g + j - 4 otherwise, and V is
-// staged in the same order.
+// is key 4 g + j for j < 4 and key 16 + 4 g + j - 4 otherwise, and the V
+// operand is read in that order.
 //
 // LDS: K and V rows as bf16 in key order, 256 bytes a row, their 16-byte
 // chunks XOR-swizzled by row.  V is transposed on the way out

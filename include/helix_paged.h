@@ -266,7 +266,8 @@ int helix_paged_attention_out(const float* query, size_t q_heads, size_t queries
  * several workgroups) and a call with several tail rows (a prefill chunk)
  * runs the exact fp32 matrix-core prefill kernel plus a normalisation
  * launch; both use a device scratch the library keeps per (device, stream),
- * allocated or grown on first use.  Every other call runs the exact scalar
+ * allocated or grown on first use.  Other calls with head sizes up to 256 run
+ * one fp32 matrix-core kernel without scratch, the rest the exact scalar
  * kernel. */
 int helix_paged_attention_with_tail_out(const float* query, size_t q_heads, size_t tail_tokens,
                                         size_t key_dim, const float* key_blocks,
