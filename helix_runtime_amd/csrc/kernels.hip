@@ -432,9 +432,9 @@ __device__ __forceinline__ float exp2_ratio(float a, float b) {
 
 // The same with v_exp_f32 directly: results below 2^-126 flush to zero, far
 // under the tolerance of a probability normalised by a sum >= 1.  Used by
-// the stream kernel on bf16 and fp8 pages, whose time follows the
-// instruction count per page (it saves exp2f's subnormal-range fix-up, four
-// instructions per call).
+// the matrix-core decode of bf16 and fp8 pages and the stream wavefronts
+// beside a cascade prefix, whose time follows the instruction count per page
+// (it saves exp2f's subnormal-range fix-up, four instructions per call).
 __device__ __forceinline__ float exp2_ratio_raw(float a, float b) {
   return a == b ? 1.0f : __builtin_amdgcn_exp2f(a - b);
 }
@@ -1014,12 +1014,11 @@ __device__ __forceinline__ void decode_stream_body(
   constexpr int DUPB = G >= 4 ? 0 : (G == 2 ? 1 : 2);
   constexpr int NV = 8 * G;
   constexpr int kStage = kStreamStage;
-  // fp8 and bf16 pages, and stream wavefronts beside prefix workgroups: the
-  // raw exp2 and a ballot for the rescale test (measured: config 3 fp8
-  // 110.7 -> 108.4 us per layer, config 4 fused cascade 79.9 -> 79.3 us;
-  // bf16 within its box-to-box spread; the plain fp32 stream kernel, bound
-  // by HBM, showed no gain and keeps exp2f).
-  constexpr bool LEAN = PF != 0 || SHARED_BLOCK;
+  // Stream wavefronts beside prefix workgroups (on every page type): the raw
+  // exp2 and a ballot for the rescale test (128 forks of one prompt, fp32
+  // pages, 79.9 -> 79.3 us; the plain stream kernel, bound by HBM, showed no
+  // gain and keeps exp2f).
+  constexpr bool LEAN = SHARED_BLOCK;
   auto& s_p = sh.p;
   auto& s_head = sh.head;
   auto& s_res_o = sh.res_o;
