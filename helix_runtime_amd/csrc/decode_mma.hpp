@@ -43,10 +43,17 @@
 // formed at once, one per lane, and read back with v_readlane: no scalar
 // load or division stands between a page and the next one's loads.
 //
-// Special values.  The split can only go wrong by giving NaN where fp32 does
-// not (a zero term times an infinite element).  Every such NaN reaches the
-// range's sum or outputs, and a range that ends with a NaN there is
-// recomputed by the wavefront with fp32 arithmetic before it is published.
+// Special values.  A finite element times the three terms sums to what it
+// gives in one product, and a NaN or an infinite operand of the split stays
+// one in its high term: fp8 pages, which hold no infinities, need nothing
+// more.  A bf16 page's infinity times a term that is zero is a NaN that fp32
+// does not give.  Every such NaN reaches the range's sum or outputs, so a
+// range of bf16 pages that ends with a NaN there is scanned for infinities
+// and, if it has one, computed again with fp32 arithmetic before it is
+// published.  One layer of the 64 sequences above, one of them with a NaN
+// element: bf16 pages 119 -> 122 us, fp8 pages 72 -> 73 (1100 and 730 when
+// every such range was computed again, row by row); with an infinite key,
+// bf16 pages 201 us.
 #pragma once
 
 #include "bf16.hpp"
@@ -502,79 +509,184 @@ __device__ __forceinline__ void decode_mma_body(
     a.part_ml[((unit + wave) * G + h) * 2 + 1] = lh;
   };
 
-  // The range [unit_p, last] of the unit in fp32, one head after another;
-  // the lane holds dims 2 lane and 2 lane + 1.
-  auto redo = [&](int b, int kvh, int last, bool tailed, bool complete) {
+  // The range [unit_p, last] of a bf16 unit again, in fp32 (Special values,
+  // above): first a scan of its elements for infinities, then, if it has any,
+  // the heads of a page together, the next page on its way meanwhile.  A lane
+  // holds dims 32 (lane & 3) .. + 31 of key lane / 4 for the scores and dims
+  // 2 lane, 2 lane + 1 of every value row.  `lds_q`: the finished page's
+  // stage.  Returns false, with nothing written, if the range has no
+  // infinity.
+  auto redo = [&](int b, int kvh, int last, bool tailed, bool complete, unsigned char* lds_q) {
     const int hist = clamp_length(scalar_read(a.lengths + b), a.max_blocks);
+    const int pages = last - unit_p + (tailed ? 0 : 1);  // without the tail row
+    const int first = unit_p + a.first_page;
+    auto page_at = [&](int i) {  // byte offset of the i-th page in the pools
+      const std::uint32_t phys =
+          scalar_read(a.tables + static_cast<std::size_t>(b) * a.max_blocks + first + i);
+      return (static_cast<std::size_t>(phys) * a.kv_heads + kvh) * Geo::kPage;
+    };
+    const auto* const kpool = reinterpret_cast<const unsigned char*>(a.key_pool);
+    const auto* const vpool = reinterpret_cast<const unsigned char*>(a.value_pool);
+    // Two elements of the tail row on the page grid (rows at any 4-byte
+    // address).
+    const std::size_t tail_row = (static_cast<std::size_t>(b) * a.kv_heads + kvh) * D;
+    auto rounded = [](const float* row) { return bf16_pack(row[0], row[1]); };
+
+    // Smallest distance of any element (16 bits, sign off) from infinity.
+    using Pair = unsigned short __attribute__((ext_vector_type(2)));
+    Pair least = {0xffff, 0xffff};
+    auto scan = [&](unsigned w) {
+      least = __builtin_elementwise_min(
+          least, __builtin_bit_cast(Pair, (w & 0x7fff7fffu) ^ 0x7f807f80u));
+    };
+    // (Rows past the history count too: that only costs the second pass.)
+    constexpr int SP = G == 8 ? 1 : 2;  // pages at a time, as the registers allow
 #pragma unroll 1
-    for (int h = 0; h < G; ++h) {
-      const float2 q = reinterpret_cast<const float2*>(
-          a.query + (static_cast<std::size_t>(b) * a.q_heads + kvh * G + h) * D)[lane];
-      float2 o = make_float2(0.f, 0.f);
-      float rm = -INFINITY, rl = 0.0f;
-#pragma unroll 1
-      for (int p = unit_p; p <= last; ++p) {
-        const bool tail = tailed && p == last;
-        const int rows = tail ? 1 : min(P, hist - (p + a.first_page) * P);
-        const std::uint32_t phys =
-            tail ? 0
-                 : scalar_read(a.tables + static_cast<std::size_t>(b) * a.max_blocks + p +
-                               a.first_page);
-        const std::size_t page = (static_cast<std::size_t>(phys) * a.kv_heads + kvh) * P * D;
-#pragma unroll 1
-        for (int r = 0; r < rows; ++r) {
-          float2 k, v;
-          if (tail) {
-            const std::size_t row = (static_cast<std::size_t>(b) * a.kv_heads + kvh) * D;
-            k = reinterpret_cast<const float2*>(a.tail_key + row)[lane];
-            v = reinterpret_cast<const float2*>(a.tail_value + row)[lane];
-            if constexpr (FP8) {
-              k = make_float2(fp8_value(fp8_code(k.x / a.k_scale), 1.0f),
-                              fp8_value(fp8_code(k.y / a.k_scale), 1.0f));
-              v = make_float2(fp8_value(fp8_code(v.x / a.v_scale), 1.0f),
-                              fp8_value(fp8_code(v.y / a.v_scale), 1.0f));
-            } else {
-              k = make_float2(bf16_value(bf16_round(k.x)), bf16_value(bf16_round(k.y)));
-              v = make_float2(bf16_value(bf16_round(v.x)), bf16_value(bf16_round(v.y)));
-            }
-          } else if constexpr (FP8) {
-            const std::size_t e = page / 2 + r * 64 + lane;
-            const unsigned kw = reinterpret_cast<const unsigned short*>(a.key_pool)[e];
-            const unsigned vw = reinterpret_cast<const unsigned short*>(a.value_pool)[e];
-            k = make_float2(fp8_value(kw & 0xffu, 1.0f), fp8_value(kw >> 8, 1.0f));
-            v = make_float2(fp8_value(vw & 0xffu, 1.0f), fp8_value(vw >> 8, 1.0f));
-          } else {
-            const std::size_t e = page / 2 + r * 64 + lane;
-            const unsigned kw = reinterpret_cast<const unsigned*>(a.key_pool)[e];
-            const unsigned vw = reinterpret_cast<const unsigned*>(a.value_pool)[e];
-            k = make_float2(__uint_as_float(kw << 16), __uint_as_float(kw & 0xffff0000u));
-            v = make_float2(__uint_as_float(vw << 16), __uint_as_float(vw & 0xffff0000u));
-          }
-          float s = q.x * k.x + q.y * k.y;
+    for (int i = 0; i < pages; i += SP) {
+      uint4 x[SP][2 * Geo::kLoads];
 #pragma unroll
-          for (int x = 32; x > 0; x >>= 1) s += __shfl_xor(s, x, 64);
-          s *= a.qscale;
-          const float mn = fmaxf(rm, s);
-          const float alpha = exp2_ratio_raw(rm, mn);
-          const float pr = exp2_ratio_raw(s, mn);
-          rl = rl * alpha + pr;
-          o.x = o.x * alpha + pr * v.x;
-          o.y = o.y * alpha + pr * v.y;
-          rm = mn;
+      for (int n = 0; n < SP; ++n) {
+        const std::size_t off = page_at(min(i + n, pages - 1)) + static_cast<std::size_t>(lane) * 16;
+#pragma unroll
+        for (int j = 0; j < Geo::kLoads; ++j) {
+          x[n][2 * j] = *reinterpret_cast<const uint4*>(kpool + off + j * 1024);
+          x[n][2 * j + 1] = *reinterpret_cast<const uint4*>(vpool + off + j * 1024);
         }
       }
-      float sc = FP8 ? a.v_scale : 1.0f;
-      if (complete) sc = rm == -INFINITY ? NAN : sc / rl;
-      reinterpret_cast<float2*>(result_row(b, kvh, complete, h))[lane] =
-          make_float2(o.x * sc, o.y * sc);
-      if (!complete && lane == 0) write_ml(b, kvh, h, rm, rl);
+#pragma unroll
+      for (int n = 0; n < SP * 2 * Geo::kLoads; ++n) {
+        const uint4 w = x[n % SP][n / SP];
+        scan(w.x), scan(w.y), scan(w.z), scan(w.w);
+      }
     }
-    // Nothing of this path is pending afterwards: the compiler would
-    // otherwise wait in the page loop for registers that are loaded here.
-    __builtin_amdgcn_s_waitcnt(0);
+    if (tailed) {
+      scan(rounded(a.tail_key + tail_row + 2 * lane));
+      scan(rounded(a.tail_value + tail_row + 2 * lane));
+    }
+    if (__ballot(least[0] == 0 || least[1] == 0) == 0) return false;
+
+    // Scaled query rows in LDS, 36 floats apart per 32 dims: the four lanes of
+    // a key read distinct banks.
+    const float* const rows = a.query + (static_cast<std::size_t>(b) * a.q_heads + kvh * G) * D;
+    float* const q = reinterpret_cast<float*>(lds_q);
+    for (int h = 0; h < G; ++h) {
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const int d = lane + 64 * e;
+        q[h * 144 + (d >> 5) * 36 + (d & 31)] = rows[h * D + d] * a.qscale;
+      }
+    }
+    stream_sync<true>();
+    const int steps = pages + (tailed ? 1 : 0);
+    constexpr int HG = G < 4 ? G : 4;  // heads at a time, as the registers allow
+#pragma unroll 1
+    for (int h0 = 0; h0 < G; h0 += HG) {
+      float o[HG][2], rm[HG], rl[HG];
+#pragma unroll
+      for (int h = 0; h < HG; ++h) {
+        o[h][0] = o[h][1] = rl[h] = 0.0f;
+        rm[h] = -INFINITY;
+      }
+      uint4 k[4];
+      unsigned v[P];
+      auto load_keys = [&](int i) {
+        if (i < pages) {
+          const unsigned char* const src = kpool + page_at(i) + lane * 64;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) k[j] = *reinterpret_cast<const uint4*>(src + j * 16);
+        } else {
+          const float* const src = a.tail_key + tail_row + 32 * (lane & 3);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            k[j] = make_uint4(rounded(src + 8 * j), rounded(src + 8 * j + 2),
+                              rounded(src + 8 * j + 4), rounded(src + 8 * j + 6));
+          }
+        }
+      };
+      auto load_values = [&](int i) {
+        if (i < pages) {
+          const unsigned char* const src = vpool + page_at(i) + lane * 4;
+#pragma unroll
+          for (int r = 0; r < P; ++r) {
+            v[r] = *reinterpret_cast<const unsigned*>(src + r * Geo::kRow);
+          }
+        } else {
+          v[0] = rounded(a.tail_value + tail_row + 2 * lane);
+        }
+      };
+      load_keys(0);
+      load_values(0);
+#pragma unroll 1
+      for (int i = 0; i < steps; ++i) {
+        const int valid = i == pages ? 1 : min(P, hist - (first + i) * P);
+        float s[HG];
+#pragma unroll
+        for (int h = 0; h < HG; ++h) {
+          s[h] = 0.0f;
+          const float* const qr = q + (h0 + h) * 144 + (lane & 3) * 36;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const float4 x0 = *reinterpret_cast<const float4*>(qr + 8 * j);
+            const float4 x1 = *reinterpret_cast<const float4*>(qr + 8 * j + 4);
+            const float4 k0 = bf16_widen(k[j].x, k[j].y);
+            const float4 k1 = bf16_widen(k[j].z, k[j].w);
+            s[h] += x0.x * k0.x + x0.y * k0.y + x0.z * k0.z + x0.w * k0.w;
+            s[h] += x1.x * k1.x + x1.y * k1.y + x1.z * k1.z + x1.w * k1.w;
+          }
+          s[h] += dpp<kDppQuadXor1>(s[h]);
+          s[h] += dpp<kDppQuadXor2>(s[h]);
+          // One head's query words in registers at a time.
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        if (i + 1 < steps) load_keys(i + 1);
+        const bool seen = (lane >> 2) < valid;
+#pragma unroll
+        for (int h = 0; h < HG; ++h) {
+          // (A key's four lanes hold the same bits.)
+          float mn = seen ? s[h] : -INFINITY;
+          mn = fmaxf(mn, dpp<kDppRowHalfMirror>(mn));
+          mn = fmaxf(mn, dpp<kDppRowRor8>(mn));
+          mn = fmaxf(prefill_detail::row_max(mn), rm[h]);
+          const float alpha = exp2_ratio_raw(rm[h], mn);
+          const float p = seen ? exp2_ratio_raw(s[h], mn) : 0.0f;
+          float sum = p;
+          sum += dpp<kDppRowHalfMirror>(sum);
+          sum += dpp<kDppRowRor8>(sum);
+          rl[h] = rl[h] * alpha + prefill_detail::row_sum(sum);
+          rm[h] = mn;
+          s[h] = p;
+          o[h][0] *= alpha;
+          o[h][1] *= alpha;
+        }
+#pragma unroll
+        for (int r = 0; r < P; ++r) {
+          if (r < valid) {
+            const float v0 = __uint_as_float(v[r] << 16), v1 = __uint_as_float(v[r] & 0xffff0000u);
+#pragma unroll
+            for (int h = 0; h < HG; ++h) {
+              const float p =
+                  __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(s[h]), 4 * r));
+              o[h][0] += p * v0;
+              o[h][1] += p * v1;
+            }
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        if (i + 1 < steps) load_values(i + 1);
+      }
+#pragma unroll
+      for (int h = 0; h < HG; ++h) {
+        const float sc = !complete ? 1.0f : rm[h] == -INFINITY ? NAN : 1.0f / rl[h];
+        float* const row = result_row(b, kvh, complete, h0 + h) + 2 * lane;
+        row[0] = o[h][0] * sc;
+        row[1] = o[h][1] * sc;
+        if (!complete && lane == 0) write_ml(b, kvh, h0 + h, rm[h], rl[h]);
+      }
+    }
+    return true;
   };
 
-  auto finalize = [&](const PageInFlight& d) {
+  auto finalize = [&](const PageInFlight& d, unsigned char* stage) {
     const int b = d.unit % a.batch, kvh = d.unit / a.batch;
     const float lt = prefill_detail::row_sum(l);
     bool nan = !(lt < INFINITY);
@@ -591,24 +703,31 @@ __device__ __forceinline__ void decode_mma_body(
           x += dpp<kDppRowRor4>(x);
         }
         acc[dt][i] = x;
-        nan = nan || isnan(x);
+        if constexpr (!FP8) nan = nan || isnan(x);
       }
     }
     const bool tailed = (d.meta & kPageTail) != 0;
     // With a cascade prefix every unit also has a prefix partial to merge.
     const bool complete = a.first_page == 0 && unit_p == 0 && tailed;
-    if (!unit_bad && __ballot(nan && head < G) != 0) {
-      redo(b, kvh, d.p, tailed, complete);
-      return;
+    if constexpr (!FP8) {
+      if (!unit_bad && __ballot(nan && head < G) != 0) {
+        const bool redone = redo(b, kvh, d.p, tailed, complete, stage);
+        // Nothing of this path is pending afterwards: the compiler would
+        // otherwise wait in the page loop for registers that are loaded here.
+        __builtin_amdgcn_s_waitcnt(0);
+        if (redone) return;
+      }
     }
     float sc = FP8 ? a.v_scale : 1.0f;
     if (complete) sc = m == -INFINITY || unit_bad ? NAN : sc / lt;
     if (col < G) {
-      float4* row = reinterpret_cast<float4*>(result_row(b, kvh, complete, col));
+      // (The output, too, may lie at any 4-byte address.)
+      using Row4 = float __attribute__((ext_vector_type(4), aligned(4)));
+      Row4* row = reinterpret_cast<Row4*>(result_row(b, kvh, complete, col));
 #pragma unroll
       for (int dt = 0; dt < 8; ++dt) {
-        row[4 * dt + grp] = make_float4(acc[dt][0] * sc, acc[dt][1] * sc, acc[dt][2] * sc,
-                                        acc[dt][3] * sc);
+        row[4 * dt + grp] = Row4{acc[dt][0] * sc, acc[dt][1] * sc, acc[dt][2] * sc,
+                                 acc[dt][3] * sc};
       }
       if (!complete && grp == 0) write_ml(b, kvh, col, m, unit_bad ? NAN : lt);
     }
@@ -798,7 +917,7 @@ __device__ __forceinline__ void decode_mma_body(
     } else {
       values(std::false_type{});
     }
-    if ((d.meta & kPageEnd) != 0) finalize(d);
+    if ((d.meta & kPageEnd) != 0) finalize(d, base);
   };
 
 #pragma unroll
