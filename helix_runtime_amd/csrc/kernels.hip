@@ -1615,40 +1615,47 @@ void cascade_decode_kernel(
       stream_lds(sh.stream[w]));
 }
 
-// Combines the partials of units that span several stream wavefronts.  A
-// workgroup takes HB query heads of one unit (kv head major: kvh * batch +
-// b): per head, group g of NG groups of 32 threads takes the unit's partials
-// g, g + NG, ... with L of them loaded at once, thread d4 of a group 4
-// output dims; the groups' results are combined through LDS.
-template <int G, int NG, int HB, int L>
-__global__ __launch_bounds__(HB * NG * 32) void decode_stream_merge_kernel(DecodeKernelArgs a) {
+// Combines the partials of units that span several stream wavefronts.  A row
+// (query head of a unit, kv head major: kvh * batch + b) has HV groups of 32
+// lanes (half-wavefronts); each takes every HV-th partial, L of them loaded at
+// once, a lane 4 output dims.  HV = 1 and 2: a workgroup takes the G rows of a
+// unit and nothing passes through LDS; more: a workgroup is one row, and one
+// whose partials two halves can load at once is left to its first wavefront.
+template <int G, int HV>
+__global__ __launch_bounds__(HV <= 2 ? G * HV * 32 : HV * 32) void decode_stream_merge_kernel(
+    DecodeKernelArgs a) {
   constexpr int D = 128;
-  constexpr int kBlocks = G / HB;  // workgroups per unit
-  __shared__ __align__(16) float4 s_o[HB][NG][32];
-  __shared__ float s_ml[HB][NG][2];
-  const int unit = static_cast<int>(blockIdx.x) / kBlocks;
-  const int hb = static_cast<int>(threadIdx.x) / (NG * 32);
-  const int h = static_cast<int>(blockIdx.x) % kBlocks * HB + hb;
+  constexpr int L = HV == 1 || HV == 16 ? 8 : 4;  // partials on their way at once
+  constexpr int NW = HV / 2;  // wavefronts of a row
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / 64);
+  const int unit = static_cast<int>(blockIdx.x) / (HV <= 2 ? 1 : G);
+  const int h = HV == 1   ? static_cast<int>(threadIdx.x) / 32
+                : HV == 2 ? wave
+                          : static_cast<int>(blockIdx.x) % G;
+  const int w = HV <= 2 ? 0 : wave;
   const int2 seg = reinterpret_cast<const int2*>(a.segments)[unit];
   const bool cascade = a.first_page > 0;
   if (seg.y <= 1 && !cascade) return;
   const int kvh = unit / a.batch;
   const int b = unit % a.batch;
-  const int grp = static_cast<int>(threadIdx.x) / 32 % NG;
+  const int half = HV == 1 ? 0 : static_cast<int>(threadIdx.x) / 32 % 2;
   const int d4 = static_cast<int>(threadIdx.x) % 32;
   const std::size_t slot0 = static_cast<std::size_t>(unit) + seg.x;
+  // Partials: the unit's stream segments, then (cascade) its prefix chunks.
+  const int nparts = seg.y + (cascade ? a.prefix_chunks : 0);
+  const bool alone = HV <= 2 || nparts <= 2 * L;
+  if (alone && w != 0) return;
+  const int step = HV == 1 ? 1 : alone ? 2 : HV;
   float mx = -INFINITY;
   float den = 0.0f;
   float4 num = make_float4(0.f, 0.f, 0.f, 0.f);
-  // Partials: the unit's stream segments, then (cascade) its prefix chunks.
-  const int nparts = seg.y + (cascade ? a.prefix_chunks : 0);
   const long long units = static_cast<long long>(a.batch) * a.kv_heads;
-  for (int s0 = grp; s0 < nparts; s0 += NG * L) {
+  for (int s0 = 2 * w + half; s0 < nparts; s0 += step * L) {
     float ms[L], ls[L];
     float4 os[L];
 #pragma unroll
     for (int i = 0; i < L; ++i) {
-      const int s = s0 + i * NG;
+      const int s = s0 + i * step;
       const bool in = s < nparts;
       const std::size_t slot =
           !in ? slot0
@@ -1670,37 +1677,58 @@ __global__ __launch_bounds__(HB * NG * 32) void decode_stream_merge_kernel(Decod
     num.w *= sc;
 #pragma unroll
     for (int i = 0; i < L; ++i) {
-      const float w = s0 + i * NG < nparts ? exp2_ratio(ms[i], cm) : 0.0f;
-      den += w * ls[i];
-      num.x += w * os[i].x;
-      num.y += w * os[i].y;
-      num.z += w * os[i].z;
-      num.w += w * os[i].w;
+      const float wt = s0 + i * step < nparts ? exp2_ratio(ms[i], cm) : 0.0f;
+      den += wt * ls[i];
+      num.x += wt * os[i].x;
+      num.y += wt * os[i].y;
+      num.z += wt * os[i].z;
+      num.w += wt * os[i].w;
     }
     mx = cm;
   }
-  if constexpr (NG > 1) {
-    s_o[hb][grp][d4] = num;
-    if (d4 == 0) {
-      s_ml[hb][grp][0] = mx;
-      s_ml[hb][grp][1] = den;
-    }
-    __syncthreads();
-    if (grp != 0) return;
-    const int live = nparts < NG ? nparts : NG;
-    for (int g = 1; g < live; ++g) mx = fmaxf(mx, s_ml[hb][g][0]);
-    den = 0.0f;
-    num = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int g = 0; g < live; ++g) {
-      const float w = exp2_ratio(s_ml[hb][g][0], mx);
-      const float4 o = s_o[hb][g][d4];
-      den += w * s_ml[hb][g][1];
-      num.x += w * o.x;
-      num.y += w * o.y;
-      num.z += w * o.z;
-      num.w += w * o.w;
+  if constexpr (HV > 1) {
+    // The two halves (one without partials has mx = -inf and zeros).
+    const float cm = fmaxf(mx, half_xor(mx));
+    const float sc = exp2_ratio(mx, cm);
+    den *= sc;
+    num.x *= sc;
+    num.y *= sc;
+    num.z *= sc;
+    num.w *= sc;
+    den += half_xor(den);
+    num.x += half_xor(num.x);
+    num.y += half_xor(num.y);
+    num.z += half_xor(num.z);
+    num.w += half_xor(num.w);
+    mx = cm;
+  }
+  if constexpr (HV > 2) {
+    if (!alone) {
+      __shared__ __align__(16) float4 s_o[NW][32];
+      __shared__ float s_ml[NW][2];
+      if (half == 0) s_o[w][d4] = num;
+      if (threadIdx.x % 64 == 0) {
+        s_ml[w][0] = mx;
+        s_ml[w][1] = den;
+      }
+      __syncthreads();
+      if (w != 0) return;
+      // More than 2 L partials: every wavefront has had some.
+      for (int g = 1; g < NW; ++g) mx = fmaxf(mx, s_ml[g][0]);
+      den = 0.0f;
+      num = make_float4(0.f, 0.f, 0.f, 0.f);
+      for (int g = 0; g < NW; ++g) {
+        const float wt = exp2_ratio(s_ml[g][0], mx);
+        const float4 o = s_o[g][d4];
+        den += wt * s_ml[g][1];
+        num.x += wt * o.x;
+        num.y += wt * o.y;
+        num.z += wt * o.z;
+        num.w += wt * o.w;
+      }
     }
   }
+  if (half != 0) return;
   float4 r;
   if (mx == -INFINITY) {
     r = make_float4(NAN, NAN, NAN, NAN);
@@ -2596,41 +2624,76 @@ void launch_stream(const dim3& grid, hipStream_t stream, const DecodeKernelArgs&
   });
 }
 
-// The merge is bound by latency: a unit has about as many partials as the
-// launch has wavefronts over units, from a handful in a full batch to
-// hundreds for one long sequence, and one group reading those 8 at a time
-// took longer than the attention.  More groups per row cut that chain, as
-// long as the launch stays around what the CUs hold at once (2048 threads
-// each).  One layer with its merge, us, 32/8 heads unless said: one sequence
-// of 4000 tokens, fp32 65 -> 23 and fp8 58 -> 17 (27 and 21 with 8 groups);
-// 4 of 100-2000, fp32 37 -> 20; 8 x 32 heads of 128-2048 tokens (1 head per
-// row group) 40.1 -> 38.2 (8 groups; 38.4 with 4); 64 sequences, fp32 225.3
-// -> 224.3 (4 groups; 225.4 with 8); 128 forks of one prompt 62.9 with one
-// group, 64.7 with 4, 66.4 with 8; 22 of 98 tokens (8 partials each), fp32
-// 15.7 with one group, 16.1 with 8.
-template <int G>
-void launch_stream_merge_group(hipStream_t stream, const DecodeKernelArgs& k) {
-  const unsigned units = static_cast<unsigned>(k.batch) * static_cast<unsigned>(k.kv_heads);
-  const unsigned rows = units * G;
-  // No unit has more partials than pages: up to 8 are read at once anyway.
-  const bool few = k.max_blocks - k.first_page + 1 + k.prefix_chunks <= 8;
-  if (few || rows >= 4096) {
-    decode_stream_merge_kernel<G, 1, G, 8><<<units, G * 32, 0, stream>>>(k);
-  } else if (rows >= 2048) {
-    decode_stream_merge_kernel<G, 4, 1, 4><<<rows, 128, 0, stream>>>(k);
-  } else if (rows >= 512) {
-    decode_stream_merge_kernel<G, 8, 1, 4><<<rows, 256, 0, stream>>>(k);
+// Most partials that a unit of the launch can have: a unit of n pages in
+// ranges of C pages spans ceil((n - 1) / C) + 1 of them at most.  Without
+// known lengths (C = 1) as many as the table has pages.
+std::size_t most_partials(const DecodeArgs& a, std::size_t waves, int prefix_chunks) {
+  const bool known = a.longest_pages != 0;
+  const std::size_t pages = (known ? a.longest_pages : a.max_blocks) - a.shared_pages;  // + the tail
+  const std::size_t total =
+      known ? (a.total_pages - a.batch * a.shared_pages + a.batch) * a.kv_heads : 0;
+  const std::size_t C = known ? (total + waves - 1) / waves : 1;
+  return (pages + C - 1) / C + 1 + static_cast<std::size_t>(prefix_chunks);
+}
+
+template <int G, int HV>
+void launch_merge_variant(unsigned units, hipStream_t stream, const DecodeKernelArgs& k) {
+  if constexpr (HV <= 2) {
+    decode_stream_merge_kernel<G, HV><<<units, G * HV * 32, 0, stream>>>(k);
   } else {
-    decode_stream_merge_kernel<G, 16, 1, 4><<<rows, 512, 0, stream>>>(k);
+    decode_stream_merge_kernel<G, HV><<<units * G, HV * 32, 0, stream>>>(k);
   }
 }
 
-hipError_t launch_stream_merge(std::size_t group, hipStream_t stream, const DecodeKernelArgs& k) {
+// The merge is bound by latency: the chain of loads of the unit with the most
+// partials (one long sequence of a ragged batch can have hundreds), and the
+// dispatch of the launch's wavefronts (about 0.2 us per 1000).  Up to 8
+// partials one or two half-wavefronts a row read in one round, two with half
+// the loads each; past that the lanes per row follow the row count.  One layer
+// with its merge, us, fp32 pages, 32/8 heads, with 1 / 4 / 8 / 16
+// half-wavefronts a row:
+//   128 rows, 4 of 900 tokens: 26.4 with 1, 17.1 with 16
+//   256 rows, one of 8000 tokens among 100s: 53.5 with 1, 25.5 with 16
+//   1024 rows, the same: 55.9 / 37.8 / 33.3 / 32.4; all 98: 17.0 / 17.2 / 17.2 / 17.2
+//   2016 rows, the same: 50.6 / 36.7 / 32.5 / 31.2
+//   2048 rows, the same: 52.7 / 39.1 / 37.5 / 33.6; all 98: 18.9 / 19.2 / 19.2 / 19.8
+//   3200 rows, all 98: 24.9 / 25.3 / 25.6 / 26.8
+//   4096 rows, the same: 54.7 / 46.6 / 43.2 / 43.8; all 98: 27.9 / 28.7 / 29.3 / 30.7;
+//     forks of a 1032-token prompt: 63.9 / 64.9 / 65.3 / 66.5
+// Two half-wavefronts: 512 rows of 8 partials 13.5 with 1, 12.5 with 2; 1024
+// of 8 17.0, 16.9; 32 of 5 10.7, 11.0; 2048 of 5 18.9, 19.0.  With one head
+// per unit a half-wavefront leaves the other half empty, so two cost no
+// dispatch: better at few rows and with many partials (32/32 heads, 8 of 98
+// tokens 13.9 with 1, 13.7 with 2; 128, one of 8000 among 100s, 126.2, 123.5),
+// worse where a full launch has few (32 of 60: 18.9, 19.2).
+template <int G>
+void launch_stream_merge_group(hipStream_t stream, const DecodeKernelArgs& k, std::size_t most) {
+  const unsigned units = static_cast<unsigned>(k.batch) * static_cast<unsigned>(k.kv_heads);
+  const unsigned rows = units * G;
+  if (most <= 8) {
+    if (rows < (most > 5 ? 2048 : G == 1 ? 512 : 0)) {
+      launch_merge_variant<G, 2>(units, stream, k);
+    } else {
+      launch_merge_variant<G, 1>(units, stream, k);
+    }
+  } else if (rows >= 4096) {
+    launch_merge_variant<G, G == 1 ? 2 : 1>(units, stream, k);
+  } else if (rows >= 2048) {
+    launch_merge_variant<G, 4>(units, stream, k);
+  } else if (rows >= 512) {
+    launch_merge_variant<G, 8>(units, stream, k);
+  } else {
+    launch_merge_variant<G, 16>(units, stream, k);
+  }
+}
+
+hipError_t launch_stream_merge(std::size_t group, hipStream_t stream, const DecodeKernelArgs& k,
+                               std::size_t most) {
   switch (group) {
-    case 1: launch_stream_merge_group<1>(stream, k); break;
-    case 2: launch_stream_merge_group<2>(stream, k); break;
-    case 4: launch_stream_merge_group<4>(stream, k); break;
-    case 8: launch_stream_merge_group<8>(stream, k); break;
+    case 1: launch_stream_merge_group<1>(stream, k, most); break;
+    case 2: launch_stream_merge_group<2>(stream, k, most); break;
+    case 4: launch_stream_merge_group<4>(stream, k, most); break;
+    case 8: launch_stream_merge_group<8>(stream, k, most); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -2727,7 +2790,7 @@ hipError_t launch_decode(const DecodeArgs& a, hipStream_t stream) {
           e = hipEventRecord(a.between_event, stream);
           if (e != hipSuccess) return e;
         }
-        return launch_stream_merge(group, stream, k);
+        return launch_stream_merge(group, stream, k, most_partials(a, waves, k.prefix_chunks));
       }
       if (overlap) {
         hipError_t e = hipEventRecord(a.fork_event, stream);
@@ -2769,7 +2832,7 @@ hipError_t launch_decode(const DecodeArgs& a, hipStream_t stream) {
       e = hipStreamWaitEvent(stream, a.join_event, 0);
       if (e != hipSuccess) return e;
     }
-    return launch_stream_merge(group, stream, k);
+    return launch_stream_merge(group, stream, k, most_partials(a, waves, k.prefix_chunks));
   }
   const WorkspaceLayout lay = layout_for(a.batch, a.q_heads, a.kv_heads, max_splits);
   k.part_o = reinterpret_cast<float*>(ws + lay.part_o);

@@ -135,6 +135,12 @@ struct DecodeArgs {
   std::size_t physical_blocks;
   std::size_t pages_per_split;
   std::size_t items;
+  // Stream mode: history pages of the longest sequence and of all sequences
+  // (shared ones counted for each), where the host knows them; 0: unknown.
+  // They only choose the merge's launch shape, so a captured launch may be
+  // replayed with other lengths.
+  std::size_t longest_pages = 0;
+  std::size_t total_pages = 0;
   // Optional: recorded on the stream between the main kernel and the merge
   // (measurement of the dominant kernel alone).
   hipEvent_t between_event = nullptr;

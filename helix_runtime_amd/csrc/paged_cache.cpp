@@ -519,11 +519,15 @@ void DecodeBatch::prepare(hipStream_t stream, std::size_t tokens) {
   auto* slots = reinterpret_cast<std::int64_t*>(host + align8(B * sizeof(std::int32_t)));
   auto* updates = reinterpret_cast<std::uint32_t*>(slots + B * tokens);  // host staging
   std::size_t n_updates = 0;
+  longest_pages_ = total_pages_ = 0;
   for (std::size_t i = 0; i < B; ++i) {
     const AppendPlan plan = s.manager.plan_append(sequences_[i], tokens);
     s.manager.commit_append(plan);
     lengths[i] = static_cast<std::int32_t>(plan.old_length);
     host_lengths_[i] = lengths[i];
+    const std::size_t pages = (plan.old_length + c.block_tokens - 1) / c.block_tokens;
+    longest_pages_ = std::max(longest_pages_, pages);
+    total_pages_ += pages;
     for (std::size_t t = 0; t < tokens; ++t) {
       slots[i * tokens + t] = static_cast<std::int64_t>(plan.slot(t, c.block_tokens));
     }
@@ -719,6 +723,8 @@ void DecodeBatch::attention_layer(std::size_t layer, const float* query, const f
   a.physical_blocks = c.physical_blocks;
   a.pages_per_split = pages_per_split_;
   a.items = items_;
+  a.longest_pages = longest_pages_;
+  a.total_pages = total_pages_;
   a.between_event = between_event_;
   a.shared_pages = shared_pages_;
   a.page_type = state_->page_type;

@@ -228,6 +228,9 @@ private:
   std::size_t max_blocks_;
   std::size_t pages_per_split_;
   std::size_t items_ = 0;      // work items of the prepared step
+  // History pages of its longest sequence and of all.
+  std::size_t longest_pages_ = 0;
+  std::size_t total_pages_ = 0;
   std::vector<std::int32_t> host_lengths_;
   DeviceBuffer tables_;
   DeviceBuffer step_;       // lengths [B] int32 | slots [B, tokens] int64 | updates
