@@ -11,14 +11,19 @@
 // 64 v + 4 c .. + 3 (c = lane % 16) for P.V, each a 16-byte load when rows
 // are aligned.  The scores come out with 4 keys of one query row per lane,
 // which is the P.V operand as it stands.  No scratch: the raw scores
-// (log2 domain) wait in the caller's score workspace and each lane turns its
-// own entries into probabilities once the row's maximum and sum are known.
+// (log2 domain) wait in the lane's registers where a wavefront has one tile
+// (up to 256 keys, 128 past 64 dims), else in the caller's score workspace, and
+// each lane turns its own entries into probabilities once the row's maximum
+// and sum are known.
 //
 // The scalar kernel it replaces gave one query row to a workgroup and one
 // key to a thread, so a wavefront's 64 loads touched 64 rows and every row
 // re-read all of K and V: latency-bound.  8 heads of 64 dims, 128 query rows
 // over 1024 keys: 390 us before, 27 us now; one row of the same 143 -> 23 us;
-// 16/4 heads of 96 dims, 160 rows over 1660 keys 2.0 ms -> 66 us.
+// 16/4 heads of 96 dims, 160 rows over 1660 keys 2.0 ms -> 66 us.  A call of
+// a few keys is a chain of latencies: 4 heads of 16 dims over 65 keys 8.0 us for
+// the scalar kernel, 8.2 with the scores through the workspace, 5.8 as it is
+// (kernel alone).
 #include "kernels.hpp"
 
 #include "prefill_body.hpp"
@@ -42,6 +47,7 @@ struct TiledArgs {
   int key_dim, value_dim, block_tokens, history, tail, keys, queries, rows, offset;
   bool quad;    // history is a multiple of 4
   bool vec_ws;  // workspace rows are 16-byte aligned
+  int block_shift;  // log2 of block_tokens, or -1
   float qscale;  // log2(e) / sqrt(key_dim)
 };
 
@@ -66,8 +72,9 @@ __device__ __forceinline__ float4 load4(const float* row, int at, int dim) {
 }
 
 // DM: the head sizes' upper bound (32, 64, 128 or 256).  VEC: head sizes are
-// multiples of 4 and every tensor is 16-byte aligned.
-template <int DM, bool VEC>
+// multiples of 4 and every tensor is 16-byte aligned.  HELD: the workgroup has
+// a wavefront per tile of the keys, whose scores then stay in its registers.
+template <int DM, bool VEC, bool HELD>
 __global__ __launch_bounds__(tiled_waves<DM>() * 64) void tiled_attention_kernel(TiledArgs a) {
   constexpr int KC = DM / 16;                // 16-dim chunks of the score product
   constexpr int VC = DM <= 64 ? 1 : DM / 64; // 64-dim groups of the outputs
@@ -86,20 +93,24 @@ __global__ __launch_bounds__(tiled_waves<DM>() * 64) void tiled_attention_kernel
   const int kvh = static_cast<int>(blockIdx.y);
   const int heads = static_cast<int>(a.g.q_heads / a.g.kv_heads);
   const int T = a.queries;
+  // Division by the query count and the page size: a chain of dozens of
+  // instructions each, which the usual one row and power of two spare.
+  auto by_queries = [&](int x) { return T == 1 ? x : x / T; };
+  auto row_of = [&](int x) { return T == 1 ? 0 : x % T; };
   const int r0 = static_cast<int>(blockIdx.x) * 16;
   const int r1 = min(r0 + 16, a.rows) - 1;
 
   // This lane's query row.
   const bool live = r0 + col < a.rows;
   const int r = live ? r0 + col : r1;
-  const int t = r % T;
-  const std::size_t qrow = (static_cast<std::size_t>(kvh) * heads + r / T) * T + t;
+  const int t = row_of(r);
+  const std::size_t qrow = (static_cast<std::size_t>(kvh) * heads + by_queries(r)) * T + t;
   const int qpos = a.offset + t;
   // Keys below `all` are seen by every row of the tile, keys from `seen` on
   // by none.
-  const bool one_head = r0 / T == r1 / T;
-  const int all = min(a.keys, a.offset + (one_head ? r0 % T : 0) + 1);
-  const int seen = min(a.keys, a.offset + (one_head ? r1 % T : T - 1) + 1);
+  const bool one_head = by_queries(r0) == by_queries(r1);
+  const int all = min(a.keys, a.offset + (one_head ? row_of(r0) : 0) + 1);
+  const int seen = min(a.keys, a.offset + (one_head ? row_of(r1) : T - 1) + 1);
   float* const srow = a.g.workspace + qrow * static_cast<std::size_t>(a.keys);
 
   float4 q[KC];
@@ -120,7 +131,7 @@ __global__ __launch_bounds__(tiled_waves<DM>() * 64) void tiled_attention_kernel
     bad = false;
     if (key >= seen) return -1;
     if (key >= a.history) return -2 - (static_cast<long long>(kvh) * a.tail + (key - a.history));
-    const int page = key / a.block_tokens;
+    const int page = a.block_shift >= 0 ? key >> a.block_shift : key / a.block_tokens;
     const std::uint32_t phys = a.g.table[page];
     if (phys >= a.g.physical_blocks) {
       bad = true;
@@ -131,9 +142,10 @@ __global__ __launch_bounds__(tiled_waves<DM>() * 64) void tiled_attention_kernel
   };
 
   const int tiles = (seen + 15) / 16;
+  float4 kept = make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);  // HELD: the tile's scores
   bool bad = false;
   long long row = w < tiles ? key_row(w * 16 + col, bad) : -1;
-  for (int kt = w; kt < tiles; kt += waves) {
+  for (int kt = w; kt < tiles; kt += HELD ? tiles : waves) {
     const int k0 = kt * 16;
     const float* kp = row >= 0    ? a.g.key_blocks + row * a.key_dim
                       : row == -1 ? nullptr
@@ -175,7 +187,7 @@ __global__ __launch_bounds__(tiled_waves<DM>() * 64) void tiled_attention_kernel
     // The next tile's table entry is on its way meanwhile.
     bool next_bad = false;
     const long long next =
-        kt + waves < tiles ? key_row((kt + waves) * 16 + col, next_bad) : -1;
+        !HELD && kt + waves < tiles ? key_row((kt + waves) * 16 + col, next_bad) : -1;
 
     // Two accumulators: half the chain of dependent matrix instructions.
     v4f s0 = v4f{0.f, 0.f, 0.f, 0.f}, s1 = s0;
@@ -202,7 +214,9 @@ __global__ __launch_bounds__(tiled_waves<DM>() * 64) void tiled_attention_kernel
         if (!vis[i]) x[i] = -INFINITY;
       }
     }
-    if (live) {
+    if constexpr (HELD) {
+      kept = make_float4(x[0], x[1], x[2], x[3]);
+    } else if (live) {
       float* const dst = srow + k0 + 4 * grp;
       if (a.vec_ws && k0 + 16 <= a.keys) {
         *reinterpret_cast<float4*>(dst) = make_float4(x[0], x[1], x[2], x[3]);
@@ -331,7 +345,8 @@ __global__ __launch_bounds__(tiled_waves<DM>() * 64) void tiled_attention_kernel
     const float inv = s_fin[0][rr] == -INFINITY ? NAN : 1.0f / s_fin[1][rr];
     const int rt = r0 + rr;
     float* const dst =
-        a.g.out + ((static_cast<std::size_t>(kvh) * heads + rt / T) * T + rt % T) * a.value_dim + d;
+        a.g.out +
+        ((static_cast<std::size_t>(kvh) * heads + by_queries(rt)) * T + row_of(rt)) * a.value_dim + d;
     if constexpr (VEC) {
       *reinterpret_cast<float4*>(dst) = make_float4(o.x * inv, o.y * inv, o.z * inv, o.w * inv);
     } else {
@@ -348,7 +363,7 @@ __global__ __launch_bounds__(tiled_waves<DM>() * 64) void tiled_attention_kernel
   const float fm = s_fin[0][col];
   const float fl = s_fin[1][col];
   const bool nan_row = fm == -INFINITY || isnan(fl);
-  constexpr int kNorm = 4;
+  constexpr int kNorm = HELD ? 1 : 4;
   for (int kt = w; kt * 16 < a.keys; kt += kNorm * waves) {
     float4 x[kNorm];
     auto whole = [&](int n) {  // uniform: 16-byte entries that every row sees
@@ -358,7 +373,9 @@ __global__ __launch_bounds__(tiled_waves<DM>() * 64) void tiled_attention_kernel
 #pragma unroll
     for (int n = 0; n < kNorm; ++n) {
       const int key = (kt + n * waves) * 16 + 4 * grp;
-      if (whole(n)) {
+      if constexpr (HELD) {
+        x[n] = kept;
+      } else if (whole(n)) {
         x[n] = *reinterpret_cast<const float4*>(srow + key);
       } else {
         x[n].x = key <= qpos && key < seen ? srow[key] : -INFINITY;
@@ -418,6 +435,7 @@ hipError_t launch_tiled_attention(const GenericArgs& a, hipStream_t stream) {
   k.offset = static_cast<int>(a.offset);
   k.quad = a.history % 4 == 0;
   k.vec_ws = (a.history + a.tail) % 4 == 0 && aligned(a.workspace);
+  k.block_shift = (a.block_tokens & (a.block_tokens - 1)) == 0 ? __builtin_ctzll(a.block_tokens) : -1;
   k.qscale = 1.4426950408889634f / sqrtf(static_cast<float>(a.key_dim));
   const bool vec = a.key_dim % 4 == 0 && a.value_dim % 4 == 0 && aligned(a.query) &&
                    aligned(a.key_blocks) && aligned(a.value_blocks) && aligned(a.tail_key) &&
@@ -428,10 +446,15 @@ hipError_t launch_tiled_attention(const GenericArgs& a, hipStream_t stream) {
     constexpr int DM = decltype(dm)::value;
     constexpr int most = tiled_waves<DM>();
     const unsigned threads = 64u * static_cast<unsigned>(key_tiles < most ? key_tiles : most);
+    const bool held = key_tiles <= most;
     if (vec) {
-      tiled_attention_kernel<DM, true><<<grid, threads, 0, stream>>>(k);
+      auto* const kernel =
+          held ? tiled_attention_kernel<DM, true, true> : tiled_attention_kernel<DM, true, false>;
+      kernel<<<grid, threads, 0, stream>>>(k);
     } else {
-      tiled_attention_kernel<DM, false><<<grid, threads, 0, stream>>>(k);
+      auto* const kernel =
+          held ? tiled_attention_kernel<DM, false, true> : tiled_attention_kernel<DM, false, false>;
+      kernel<<<grid, threads, 0, stream>>>(k);
     }
   };
   const std::size_t dim = a.key_dim > a.value_dim ? a.key_dim : a.value_dim;

@@ -1,5 +1,6 @@
 """Reference-shaped attention on the fp32 matrix cores (head sizes other than
-128, other page sizes): edges of the 16-row and 16-key tiles, head sizes
+128, other page sizes): edges of the 16-row and 16-key tiles, as many key
+tiles as wavefronts and one more, head sizes
 around the 16-, 64-, 128- and 256-dim groups and not multiples of 4, grouped
 heads, key and value sizes that differ, both entry points, unaligned tensors,
 special values.
@@ -55,7 +56,11 @@ def page_rows(pool, table, hist):
     (2, 4, 64, 64, 16, 15, 5), (8, 1, 64, 64, 16, 240, 16), (2, 2, 80, 80, 16, 333, 33),
     (1, 8, 96, 64, 32, 500, 3), (2, 1, 128, 128, 8, 100, 40), (2, 1, 130, 20, 16, 31, 9),
     (1, 1, 12, 256, 16, 65, 18), (1, 2, 256, 256, 4, 129, 20), (2, 3, 65, 63, 5, 47, 31),
-    (1, 1, 32, 33, 16, 1999, 1), (2, 1, 64, 64, 16, 0, 50)])
+    (1, 1, 32, 33, 16, 1999, 1), (2, 1, 64, 64, 16, 0, 50),
+    # A wavefront per key tile, and one tile more than wavefronts.
+    (2, 1, 64, 64, 16, 255, 1), (2, 1, 64, 64, 16, 256, 1), (1, 2, 16, 16, 1, 237, 20),
+    (2, 2, 128, 128, 8, 120, 8), (2, 2, 128, 128, 8, 121, 8), (1, 1, 200, 200, 12, 127, 1),
+    (1, 1, 200, 200, 12, 128, 1)])
 @pytest.mark.parametrize("shift", [0, 1])
 def test_tail_entry_matches_64_bit(device, hkv, group, kd, vd, p, hist, t, shift):
     (q, kp, vp, tk, tv), table, d, dtable = inputs(hkv, group, kd, vd, p, hist, t,
@@ -85,8 +90,9 @@ def test_history_entry_matches_64_bit(device, kd, p, tokens, t, offset):
 
 
 @pytest.mark.parametrize("kd,p", [(64, 16), (37, 7), (160, 16)])
-def test_special_values_match_scalar_kernel(device, kd, p):
-    hist, t, hkv = 90, 20, 6
+@pytest.mark.parametrize("hist", [90, 290])
+def test_special_values_match_scalar_kernel(device, kd, p, hist):
+    t, hkv = 20, 6
     (_, _, _, _, _), table, d, dtable = inputs(hkv, 2, kd, kd, p, hist, t, 5 + kd)
     q, kp, vp, tk, tv = d
     inf, nan = float("inf"), float("nan")
