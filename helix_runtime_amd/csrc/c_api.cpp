@@ -63,25 +63,24 @@ struct AttentionShape {
 };
 
 void validate_attention(const AttentionShape& s, bool allow_empty_history, const char* op) {
-  const std::string o(op);
   check(s.physical > 0 && s.kv_heads > 0 && s.block_tokens > 0 && s.key_dim > 0,
         Status::kInvalidArgument,
-        o + ": physical block, head, token, and key dimensions must be positive");
-  check(s.value_dim > 0, Status::kInvalidArgument, o + ": value dimension must be positive");
+        op, "physical block, head, token, and key dimensions must be positive");
+  check(s.value_dim > 0, Status::kInvalidArgument, op, "value dimension must be positive");
   check(s.q_heads > 0 && s.q_heads % s.kv_heads == 0, Status::kInvalidArgument,
-        o + ": query heads must be a positive multiple of the key/value heads");
+        op, "query heads must be a positive multiple of the key/value heads");
   check(s.physical <= std::numeric_limits<std::uint32_t>::max(), Status::kInvalidArgument,
-        o + ": physical block capacity must fit the uint32 block-ID representation");
+        op, "physical block capacity must fit the uint32 block-ID representation");
   check(allow_empty_history || s.history != 0, Status::kInvalidArgument,
-        o + ": KV token count must be positive");
+        op, "KV token count must be positive");
   const std::size_t required = s.history == 0 ? 0 : 1 + (s.history - 1) / s.block_tokens;
   check(s.logical == required, Status::kInvalidArgument,
-        o + ": block table length must exactly cover the logical KV token range");
+        op, "block table length must exactly cover the logical KV token range");
   check(s.offset <= s.keys, Status::kInvalidArgument,
-        o + ": query position offset exceeds the KV token count");
+        op, "query position offset exceeds the KV token count");
   check(s.queries <= s.keys - s.offset, Status::kInvalidArgument,
-        o + ": query range extends beyond the KV token count");
-  check(s.value_dim <= 1024, Status::kUnsupported, o + ": value dimension above 1024");
+        op, "query range extends beyond the KV token count");
+  check(s.value_dim <= 1024, Status::kUnsupported, op, "value dimension above 1024");
 }
 
 // Anchor pool of a prefix cache over the device cache: its state under the
@@ -465,18 +464,17 @@ bool validate_reference_buffers(const AttentionShape& s, const float* query,
                                 const float* tail_value, const float* output,
                                 const float* workspace, std::size_t workspace_elements,
                                 const char* op) {
-  const std::string o(op);
   const std::size_t ws = mul(mul(s.q_heads, s.queries), s.keys);
   check(workspace_elements == ws, Status::kInvalidArgument,
-        o + ": score workspace shape does not match [heads, queries, kv tokens]");
+        op, "score workspace shape does not match [heads, queries, kv tokens]");
   if (s.queries == 0) return false;
   check(query != nullptr && output != nullptr && workspace != nullptr, Status::kInvalidArgument,
-        o + ": query, output and workspace must be non-null device pointers");
+        op, "query, output and workspace must be non-null device pointers");
   check(s.history == 0 || (key_blocks != nullptr && value_blocks != nullptr &&
                            block_table != nullptr),
-        Status::kInvalidArgument, o + ": key/value blocks and block table must be non-null");
+        Status::kInvalidArgument, op, "key/value blocks and block table must be non-null");
   check(s.tail == 0 || (tail_key != nullptr && tail_value != nullptr), Status::kInvalidArgument,
-        o + ": tail key and value must be non-null");
+        op, "tail key and value must be non-null");
   const std::size_t qb = mul(ws / s.keys, s.key_dim) * sizeof(float);
   const std::size_t ob = mul(ws / s.keys, s.value_dim) * sizeof(float);
   const std::size_t wb = ws * sizeof(float);
@@ -485,40 +483,41 @@ bool validate_reference_buffers(const AttentionShape& s, const float* query,
   const std::size_t vb = mul(page, s.value_dim) * sizeof(float);
   const std::size_t tkb = mul(mul(s.kv_heads, s.tail), s.key_dim) * sizeof(float);
   const std::size_t tvb = mul(mul(s.kv_heads, s.tail), s.value_dim) * sizeof(float);
-  check(!overlap(query, qb, output, ob), Status::kInvalidArgument, o + ": output must not alias query");
+  check(!overlap(query, qb, output, ob), Status::kInvalidArgument, op, "output must not alias query");
   check(!overlap(key_blocks, kb, output, ob), Status::kInvalidArgument,
-        o + ": output must not alias key blocks");
+        op, "output must not alias key blocks");
   check(!overlap(value_blocks, vb, output, ob), Status::kInvalidArgument,
-        o + ": output must not alias value blocks");
+        op, "output must not alias value blocks");
   check(!overlap(tail_key, tkb, output, ob), Status::kInvalidArgument,
-        o + ": output must not alias tail key");
+        op, "output must not alias tail key");
   check(!overlap(tail_value, tvb, output, ob), Status::kInvalidArgument,
-        o + ": output must not alias tail value");
+        op, "output must not alias tail value");
   check(!overlap(query, qb, workspace, wb), Status::kInvalidArgument,
-        o + ": score workspace must not alias query");
+        op, "score workspace must not alias query");
   check(!overlap(key_blocks, kb, workspace, wb), Status::kInvalidArgument,
-        o + ": score workspace must not alias key blocks");
+        op, "score workspace must not alias key blocks");
   check(!overlap(value_blocks, vb, workspace, wb), Status::kInvalidArgument,
-        o + ": score workspace must not alias value blocks");
+        op, "score workspace must not alias value blocks");
   check(!overlap(tail_key, tkb, workspace, wb), Status::kInvalidArgument,
-        o + ": score workspace must not alias tail key");
+        op, "score workspace must not alias tail key");
   check(!overlap(tail_value, tvb, workspace, wb), Status::kInvalidArgument,
-        o + ": score workspace must not alias tail value");
+        op, "score workspace must not alias tail value");
   check(!overlap(workspace, wb, output, ob), Status::kInvalidArgument,
-        o + ": output must not alias score workspace");
+        op, "output must not alias score workspace");
   return true;
 }
 
+// Fails as "op launch: ..." unless e is success.
+void launched(hipError_t e, const char* op) {
+  if (e != hipSuccess) helix::hip_check(e, (std::string(op) + " launch").c_str());
+}
+
+// The call (buffers validated) at any geometry.
 void run_reference_attention(const AttentionShape& s, const float* query,
                              const float* key_blocks, const float* value_blocks,
                              const std::uint32_t* block_table, const float* tail_key,
                              const float* tail_value, float* output, float* workspace,
-                             std::size_t workspace_elements, bool scalar, hipStream_t stream,
-                             const char* op) {
-  if (!validate_reference_buffers(s, query, key_blocks, value_blocks, block_table, tail_key,
-                                  tail_value, output, workspace, workspace_elements, op)) {
-    return;
-  }
+                             bool scalar, hipStream_t stream, const char* op) {
   helix::hip::GenericArgs a{};
   a.query = query;
   a.key_blocks = key_blocks;
@@ -543,7 +542,7 @@ void run_reference_attention(const AttentionShape& s, const float* query,
   const hipError_t e = !scalar && helix::hip::tiled_attention_fits(a)
                            ? helix::hip::launch_tiled_attention(a, stream)
                            : helix::hip::launch_generic(a, stream);
-  helix::hip_check(e, (std::string(op) + " launch").c_str());
+  launched(e, op);
 }
 
 // Device scratch of the reference-shaped fast routes, one buffer per
@@ -623,7 +622,7 @@ bool try_ref_decode(const AttentionShape& s, const float* query, const float* ke
   a.keys = s.keys;
   a.tail = tail;
   a.scratch = route_scratch(plan.scratch_bytes, stream, ScratchUse::kDecode);
-  helix::hip_check(hh::launch_ref_decode(a, plan, stream), (std::string(op) + " launch").c_str());
+  launched(hh::launch_ref_decode(a, plan, stream), op);
   return true;
 }
 
@@ -681,7 +680,7 @@ void run_ref_prefill(const AttentionShape& s, const float* query, const float* k
       ScratchUse::kRowStats));
   a.prob_ml = stats;
   a.prob_o = stats + ml_floats;
-  helix::hip_check(hh::launch_prefill(a, stream), (std::string(op) + " launch").c_str());
+  launched(hh::launch_prefill(a, stream), op);
 }
 
 // _with_tail_out with several tail rows: the tail is the chunk.
@@ -749,7 +748,7 @@ int helix_paged_attention_out(const float* query, size_t q_heads, size_t queries
       return;
     }
     run_reference_attention(s, query, key_blocks, value_blocks, block_table, nullptr, nullptr,
-                            output, score_workspace, workspace_elements, false, as_stream(stream), op);
+                            output, score_workspace, false, as_stream(stream), op);
   });
 }
 
@@ -762,30 +761,27 @@ void attention_with_tail(const float* query, size_t q_heads, size_t tail_tokens,
                          size_t history_tokens, const float* tail_key, const float* tail_value,
                          float* output, float* score_workspace, size_t workspace_elements,
                          helix_stream stream, bool probabilities, const char* op) {
-  check(tail_tokens != 0, Status::kInvalidArgument,
-        std::string(op) + ": tail token count must be positive");
+  check(tail_tokens != 0, Status::kInvalidArgument, op, "tail token count must be positive");
   check(history_tokens <= std::numeric_limits<std::int64_t>::max() - tail_tokens,
-        Status::kResourceExhausted,
-        std::string(op) + ": history plus tail token count overflows shape range");
+        Status::kResourceExhausted, op,
+        "history plus tail token count overflows shape range");
   AttentionShape s{q_heads, tail_tokens, key_dim, physical_blocks, kv_heads, block_tokens,
                    value_dim, logical_blocks, history_tokens, tail_tokens,
                    history_tokens + tail_tokens, history_tokens};
   validate_attention(s, true, op);
-  if (!probabilities) {
-    if (!validate_reference_buffers(s, query, key_blocks, value_blocks, block_table, tail_key,
-                                    tail_value, output, score_workspace, workspace_elements, op)) {
-      return;
-    }
-    if (try_ref_decode(s, query, key_blocks, value_blocks, block_table, tail_key, tail_value,
-                       output, score_workspace, history_tokens, true, as_stream(stream), op) ||
-        try_ref_prefill(s, query, key_blocks, value_blocks, block_table, tail_key, tail_value,
-                        output, score_workspace, as_stream(stream), op)) {
-      return;
-    }
+  if (!validate_reference_buffers(s, query, key_blocks, value_blocks, block_table, tail_key,
+                                  tail_value, output, score_workspace, workspace_elements, op)) {
+    return;
+  }
+  if (!probabilities &&
+      (try_ref_decode(s, query, key_blocks, value_blocks, block_table, tail_key, tail_value,
+                      output, score_workspace, history_tokens, true, as_stream(stream), op) ||
+       try_ref_prefill(s, query, key_blocks, value_blocks, block_table, tail_key, tail_value,
+                       output, score_workspace, as_stream(stream), op))) {
+    return;
   }
   run_reference_attention(s, query, key_blocks, value_blocks, block_table, tail_key, tail_value,
-                          output, score_workspace, workspace_elements, probabilities,
-                          as_stream(stream), op);
+                          output, score_workspace, probabilities, as_stream(stream), op);
 }
 
 }  // namespace
