@@ -11,7 +11,7 @@
 // 64 v + 4 c .. + 3 (c = lane % 16) for P.V, each a 16-byte load when rows
 // are aligned.  The scores come out with 4 keys of one query row per lane,
 // which is the P.V operand as it stands.  No scratch: the raw scores
-// (log2 domain) wait in the lane's registers where a wavefront has one tile
+// wait in the lane's registers where a wavefront has one tile
 // (up to 256 keys, 128 past 64 dims), else in the caller's score workspace, and
 // each lane turns its own entries into probabilities once the row's maximum
 // and sum are known.
@@ -48,7 +48,7 @@ struct TiledArgs {
   bool quad;    // history is a multiple of 4
   bool vec_ws;  // workspace rows are 16-byte aligned
   int block_shift;  // log2 of block_tokens, or -1
-  float qscale;  // log2(e) / sqrt(key_dim)
+  float qscale;  // 1 / sqrt(key_dim); scores of calls past HELD also times log2(e)
 };
 
 // Wavefronts of a workgroup: the merge holds one 16 x DM output tile of each
@@ -56,6 +56,30 @@ struct TiledArgs {
 template <int DM>
 constexpr int tiled_waves() {
   return DM <= 64 ? 16 : 8;
+}
+
+// exp(t) for t <= 0 (or NaN): 2^(t log2 e) with the rounding of the product
+// and of log2 e put back in first order, for scores in natural units.  Over few
+// keys this is what the outputs' error is made of (4 heads of 16 dims over 65
+// keys, mean of 12 inputs against 64 bits: 1.58e-7 with scores in units of
+// log2, 1.42e-7 so, 1.50e-7 for the scalar kernel); over many it costs 3 % and
+// the order of the sums, in which this kernel is the better one, decides.
+__device__ __forceinline__ float exp_of(float t) {
+  constexpr float kL = 1.44269502162933349609375f;  // log2 e, fp32
+  constexpr float kLow = 1.92596298909e-8f;         // what it leaves out
+  t = t < -200.0f ? -200.0f : t;  // (keeps -inf out of the correction)
+  const float hi = t * kL;
+  const float lo = fmaf(t, kLow, fmaf(t, kL, -hi));
+  const float e = __builtin_amdgcn_exp2f(hi);
+  return fmaf(e, lo * 0.693147180559945309f, e);
+}
+template <bool NATURAL>
+__device__ __forceinline__ float power(float t) {
+  return NATURAL ? exp_of(t) : __builtin_amdgcn_exp2f(t);
+}
+template <bool NATURAL>
+__device__ __forceinline__ float power_ratio(float a, float b) {
+  return NATURAL ? (a == b ? 1.0f : exp_of(a - b)) : exp2_ratio(a, b);
 }
 
 // Four consecutive floats of a row from `at` on; entries past `dim` are 0.
@@ -228,13 +252,13 @@ __global__ __launch_bounds__(tiled_waves<DM>() * 64) void tiled_attention_kernel
       }
     }
     const float mn = fmaxf(m, row_max(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]))));
-    const float alpha = exp2_ratio(m, mn);
+    const float alpha = power_ratio<HELD>(m, mn);
     if (plain && __ballot(!(fabsf(mn) < INFINITY)) == 0) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) p[i] = __builtin_amdgcn_exp2f(x[i] - mn);
+      for (int i = 0; i < 4; ++i) p[i] = power<HELD>(x[i] - mn);
     } else {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) p[i] = plain || vis[i] ? exp2_ratio(x[i], mn) : 0.0f;
+      for (int i = 0; i < 4; ++i) p[i] = plain || vis[i] ? power_ratio<HELD>(x[i], mn) : 0.0f;
     }
     l = l * alpha + ((p[0] + p[1]) + (p[2] + p[3]));
     m = mn;
@@ -316,7 +340,7 @@ __global__ __launch_bounds__(tiled_waves<DM>() * 64) void tiled_attention_kernel
     float fm = xm;
 #pragma unroll
     for (int o = 8; o > 0; o >>= 1) fm = fmaxf(fm, __shfl_xor(fm, o, 16));
-    const float wt = x < waves ? exp2_ratio(xm, fm) : 0.0f;
+    const float wt = x < waves ? power_ratio<HELD>(xm, fm) : 0.0f;
     float fl = x < waves ? wt * s_ml[x][1][rr] : 0.0f;
 #pragma unroll
     for (int o = 8; o > 0; o >>= 1) fl += __shfl_xor(fl, o, 16);
@@ -392,7 +416,7 @@ __global__ __launch_bounds__(tiled_waves<DM>() * 64) void tiled_attention_kernel
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const bool sees = key + i <= qpos && key + i < seen;
-        p[i] = nan_row ? NAN : sees ? exp2_ratio(y[i], fm) / fl : 0.0f;
+        p[i] = nan_row ? NAN : sees ? power_ratio<HELD>(y[i], fm) / fl : 0.0f;
       }
       if (whole(n)) {
         *reinterpret_cast<float4*>(srow + key) = make_float4(p[0], p[1], p[2], p[3]);
@@ -436,7 +460,6 @@ hipError_t launch_tiled_attention(const GenericArgs& a, hipStream_t stream) {
   k.quad = a.history % 4 == 0;
   k.vec_ws = (a.history + a.tail) % 4 == 0 && aligned(a.workspace);
   k.block_shift = (a.block_tokens & (a.block_tokens - 1)) == 0 ? __builtin_ctzll(a.block_tokens) : -1;
-  k.qscale = 1.4426950408889634f / sqrtf(static_cast<float>(a.key_dim));
   const bool vec = a.key_dim % 4 == 0 && a.value_dim % 4 == 0 && aligned(a.query) &&
                    aligned(a.key_blocks) && aligned(a.value_blocks) && aligned(a.tail_key) &&
                    aligned(a.tail_value) && aligned(a.out);
@@ -447,6 +470,7 @@ hipError_t launch_tiled_attention(const GenericArgs& a, hipStream_t stream) {
     constexpr int most = tiled_waves<DM>();
     const unsigned threads = 64u * static_cast<unsigned>(key_tiles < most ? key_tiles : most);
     const bool held = key_tiles <= most;
+    k.qscale = (held ? 1.0f : 1.4426950408889634f) / sqrtf(static_cast<float>(a.key_dim));
     if (vec) {
       auto* const kernel =
           held ? tiled_attention_kernel<DM, true, true> : tiled_attention_kernel<DM, true, false>;
