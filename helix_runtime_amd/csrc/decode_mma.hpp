@@ -63,9 +63,9 @@
 namespace helix::hip {
 namespace {
 
-typedef short v4s __attribute__((ext_vector_type(4)));
 typedef int v2i __attribute__((ext_vector_type(2)));
 using prefill_detail::v4f;
+using prefill_detail::v4s;
 using prefill_detail::v8bf;
 using prefill_detail::v8s;
 
@@ -131,13 +131,6 @@ __device__ __forceinline__ unsigned split_term(float x, unsigned mask1, unsigned
   t -= __uint_as_float(__float_as_uint(t) & mask2);
   const bool drop = mask1 != 0u && !(fabsf(x) < INFINITY);
   return drop ? 0u : __float_as_uint(t) >> 16;
-}
-
-// A uniform read of memory that the kernel does not write, through the
-// scalar cache.
-template <typename T>
-__device__ __forceinline__ T scalar_read(const T* p) {
-  return *(const __attribute__((address_space(4))) T*)(reinterpret_cast<std::uintptr_t>(p));
 }
 
 // Eight fp8 code values (two words) as one bf16 matrix operand.
@@ -310,7 +303,7 @@ __device__ __forceinline__ void decode_mma_body(
       }
       ub = __builtin_amdgcn_readfirstlane(ub);
       ukvh = __builtin_amdgcn_readfirstlane(ukvh);
-      uhist = clamp_length(scalar_read(a.lengths + ub), a.max_blocks);
+      uhist = clamp_length(prefill_detail::uniform_read(a.lengths + ub), a.max_blocks);
       unp = unit_pages(uhist, a.first_page);
       ubase = uniform64(ubase);
     }
@@ -478,7 +471,7 @@ __device__ __forceinline__ void decode_mma_body(
     unsigned char* page = stage + (key ? 0 : Geo::kPage);
     long long dst = -1;
     if constexpr (APPEND) {
-      const std::int64_t at = scalar_read(a.append_slots + b);
+      const std::int64_t at = prefill_detail::uniform_read(a.append_slots + b);
       if (at >= 0) dst = ((at / P * static_cast<long long>(a.kv_heads) + kvh) * P + at % P) * D;
     }
     float* const pool = key ? a.append_key_pool : a.append_value_pool;
@@ -517,12 +510,12 @@ __device__ __forceinline__ void decode_mma_body(
   // stage.  Returns false, with nothing written, if the range has no
   // infinity.
   auto redo = [&](int b, int kvh, int last, bool tailed, bool complete, unsigned char* lds_q) {
-    const int hist = clamp_length(scalar_read(a.lengths + b), a.max_blocks);
+    const int hist = clamp_length(prefill_detail::uniform_read(a.lengths + b), a.max_blocks);
     const int pages = last - unit_p + (tailed ? 0 : 1);  // without the tail row
     const int first = unit_p + a.first_page;
     auto page_at = [&](int i) {  // byte offset of the i-th page in the pools
-      const std::uint32_t phys =
-          scalar_read(a.tables + static_cast<std::size_t>(b) * a.max_blocks + first + i);
+      const std::uint32_t phys = prefill_detail::uniform_read(
+          a.tables + static_cast<std::size_t>(b) * a.max_blocks + first + i);
       return (static_cast<std::size_t>(phys) * a.kv_heads + kvh) * Geo::kPage;
     };
     const auto* const kpool = reinterpret_cast<const unsigned char*>(a.key_pool);
@@ -546,7 +539,8 @@ __device__ __forceinline__ void decode_mma_body(
       uint4 x[SP][2 * Geo::kLoads];
 #pragma unroll
       for (int n = 0; n < SP; ++n) {
-        const std::size_t off = page_at(min(i + n, pages - 1)) + static_cast<std::size_t>(lane) * 16;
+        const std::size_t off =
+            page_at(min(i + n, pages - 1)) + static_cast<std::size_t>(lane) * 16;
 #pragma unroll
         for (int j = 0; j < Geo::kLoads; ++j) {
           x[n][2 * j] = *reinterpret_cast<const uint4*>(kpool + off + j * 1024);

@@ -110,19 +110,16 @@ void prefill_redo_kernel(PrefillKernelArgs a, const std::uint32_t* __restrict__ 
   prefill_body<G, false, PF, RT>(a, tables, order, blockIdx.x, sh);
 }
 
-// Tiles per wavefront of the bf16 matrix-core prefill: one (8 wavefronts
-// of 16 rows) keeps two of the query operand's three terms (the third is
-// in LDS), the accumulators and the staging of a wavefront within 128
-// VGPRs, four wavefronts per SIMD.
-constexpr int kBmmaTilesPerWave = 1;
-
-template <int G, int PF, int RT>
-__global__ __launch_bounds__(512 / RT, 6 - 2 * RT)
+// Eight wavefronts of 16 rows keep two of the query operand's three terms
+// (the third is in LDS), the accumulators and the staging of a wavefront
+// within 128 VGPRs, four wavefronts per SIMD.
+template <int G, int PF>
+__global__ __launch_bounds__(512, 4)
 void prefill_bmma_kernel(PrefillKernelArgs a, const std::uint32_t* __restrict__ tables,
                          const std::uint32_t* __restrict__ order,
                          std::uint32_t* __restrict__ redo) {
   __shared__ PrefillBmmaShared sh;
-  prefill_body_bmma<G, PF, RT>(a, tables, order, redo, blockIdx.x, sh);
+  prefill_body_bmma<G, PF>(a, tables, order, redo, blockIdx.x, sh);
 }
 
 // fp32 pages with a redo array: the fast variant of the fp32 kernel (no
@@ -152,8 +149,7 @@ template <int G, int PF>
 void launch_bmma(const dim3& grid, hipStream_t stream, const PrefillKernelArgs& k,
                  const std::uint32_t* tables, const std::uint32_t* order,
                  std::uint32_t* redo) {
-  constexpr int BRT = kBmmaTilesPerWave;
-  prefill_bmma_kernel<G, PF, BRT><<<grid, 512 / BRT, 0, stream>>>(k, tables, order, redo);
+  prefill_bmma_kernel<G, PF><<<grid, 512, 0, stream>>>(k, tables, order, redo);
   prefill_redo_kernel<G, PF, kTilesPerWave><<<grid, 512 / kTilesPerWave, 0, stream>>>(
       k, tables, order, redo);
 }

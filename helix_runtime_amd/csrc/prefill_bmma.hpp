@@ -78,9 +78,9 @@ __device__ __forceinline__ unsigned bmma_v_at(int row, int chunk) {
 
 // A uniform read of memory that the kernel does not write, through the
 // scalar cache.
-__device__ __forceinline__ std::uint32_t uniform_read(const std::uint32_t* p) {
-  return *(const __attribute__((address_space(4))) std::uint32_t*)(
-      reinterpret_cast<std::uintptr_t>(p));
+template <typename T>
+__device__ __forceinline__ T uniform_read(const T* p) {
+  return *(const __attribute__((address_space(4))) T*)(reinterpret_cast<std::uintptr_t>(p));
 }
 
 // x = hi + mid + lo exactly (truncating splits of a finite fp32); a
@@ -133,10 +133,10 @@ __device__ __forceinline__ float bf16_bits_value(unsigned short h) {
 }
 
 // PF: 1 bf16 pages, 2 fp8 pages.  Standalone prefill only (no cascade).
-// RT: 16-row tiles per wavefront; the workgroup has 8 / RT wavefronts.
+// The workgroup has 8 wavefronts of 16 query rows each.
 // redo[block] is written for every block: 1 when the item must be redone
 // exactly.
-template <int G, int PF, int RT>
+template <int G, int PF>
 __device__ __forceinline__ void prefill_body_bmma(PrefillKernelArgs a,
                                                   const std::uint32_t* __restrict__ tables,
                                                   const std::uint32_t* __restrict__ order,
@@ -174,50 +174,38 @@ __device__ __forceinline__ void prefill_body_bmma(PrefillKernelArgs a,
   // fp8: keys are bare code values, their scale joins the score scale.
   const float qs = FP8 ? a.qscale * a.k_scale : a.qscale;
 
-  // Query operand: tile t, step s covers dims 32 s + 8 grp .. + 7 of row
-  // t * 16 + col (B operand of S^T = K Q^T), as three bf16 terms.
-  int qpos[RT];
-  std::size_t qrow[RT];
-  v8s qv[RT][2][4];
+  // Query operand: step s covers dims 32 s + 8 grp .. + 7 of row col (B operand
+  // of S^T = K Q^T), as three bf16 terms.
+  v8s qv[2][4];
+  const int r = wave * 16 + col;
+  const int head = kvh * G + r / PW;
+  const int qpos = pos0 + r % PW;
+  const bool valid = qpos < T;
+  const std::size_t qrow = ((static_cast<std::size_t>(b) * a.q_heads + head) * T + qpos) * D;
 #pragma unroll
-  for (int t = 0; t < RT; ++t) {
-    const int r = wave * (16 * RT) + t * 16 + col;
-    const int head = kvh * G + r / PW;
-    qpos[t] = pos0 + r % PW;
-    const bool valid = qpos[t] < T;
-    qrow[t] = ((static_cast<std::size_t>(b) * a.q_heads + head) * T + qpos[t]) * D;
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      float4 x0 = make_float4(0.f, 0.f, 0.f, 0.f), x1 = x0;
-      if (valid) {
-        x0 = *reinterpret_cast<const float4*>(a.query + qrow[t] + 32 * s + 8 * grp);
-        x1 = *reinterpret_cast<const float4*>(a.query + qrow[t] + 32 * s + 8 * grp + 4);
-      }
-      const float xs[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-      v8s lo;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        short h, m, l;
-        split3(xs[j] * qs, h, m, l);
-        qv[t][0][s][j] = h;
-        qv[t][1][s][j] = m;
-        lo[j] = l;
-      }
-      sh.qlo[wave * RT + t][s][lane] = __builtin_bit_cast(uint4, lo);
+  for (int s = 0; s < 4; ++s) {
+    float4 x0 = make_float4(0.f, 0.f, 0.f, 0.f), x1 = x0;
+    if (valid) {
+      x0 = *reinterpret_cast<const float4*>(a.query + qrow + 32 * s + 8 * grp);
+      x1 = *reinterpret_cast<const float4*>(a.query + qrow + 32 * s + 8 * grp + 4);
     }
+    const float xs[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+    v8s lo;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      short h, m, l;
+      split3(xs[j] * qs, h, m, l);
+      qv[0][s][j] = h;
+      qv[1][s][j] = m;
+      lo[j] = l;
+    }
+    sh.qlo[wave][s][lane] = __builtin_bit_cast(uint4, lo);
   }
 
-  v4f o[RT][8];  // O^T tiles: o[t][dt][i] = O[row t*16 + col][dim 16 dt + 4 grp + i]
+  v4f o[8];  // O^T tiles: o[dt][i] = O[row col][dim 16 dt + 4 grp + i]
 #pragma unroll
-  for (int t = 0; t < RT; ++t)
-#pragma unroll
-    for (int dt = 0; dt < 8; ++dt) o[t][dt] = v4f{0.f, 0.f, 0.f, 0.f};
-  float m[RT], l[RT];
-#pragma unroll
-  for (int t = 0; t < RT; ++t) {
-    m[t] = -INFINITY;
-    l[t] = 0.f;
-  }
+  for (int dt = 0; dt < 8; ++dt) o[dt] = v4f{0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, l = 0.f;
 
   // Staging of a 16-key half (one page) of the next 32-key block.
   // - A bf16 page wholly in the history goes straight from global memory to
@@ -229,7 +217,6 @@ __device__ __forceinline__ void prefill_body_bmma(PrefillKernelArgs a,
   //   after the other, so only one page is held in registers.  The one bf16
   //   half where the history ends inside a page is loaded when it is stored,
   //   so that the loads of the others are of one kind (chunk rows).
-  static_assert(RT == 1, "eight wavefronts stage a block");
   const int srow = tid >> 5;
   const int scol = tid & 31;
   const int uwave = __builtin_amdgcn_readfirstlane(wave);
@@ -383,67 +370,59 @@ __device__ __forceinline__ void prefill_body_bmma(PrefillKernelArgs a,
     const unsigned char* K = reinterpret_cast<const unsigned char*>(sh.k[buf]);
     const unsigned char* V = reinterpret_cast<const unsigned char*>(sh.v[buf]);
 
-    // S^T = K Q^T on the bf16 matrix cores: st[t][h] holds keys
-    // 16 h + 4 grp + i of query row t * 16 + col.
-    v4f st[RT][2];
-#pragma unroll
-    for (int t = 0; t < RT; ++t) st[t][0] = st[t][1] = v4f{0.f, 0.f, 0.f, 0.f};
+    // S^T = K Q^T on the bf16 matrix cores: st[h] holds keys
+    // 16 h + 4 grp + i of query row col.
+    v4f st[2];
+    st[0] = st[1] = v4f{0.f, 0.f, 0.f, 0.f};
     // Raised wave priority over the matrix instructions: the waves of one
     // workgroup reach them together (barriers), and the softmax and staging
     // of the other workgroup on the CU fill the gaps.
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
+      const v8bf qlo = __builtin_bit_cast(v8bf, sh.qlo[wave][s][lane]);
 #pragma unroll
-      for (int t = 0; t < RT; ++t) {
-        const v8bf qlo = __builtin_bit_cast(v8bf, sh.qlo[wave * RT + t][s][lane]);
+      for (int h = 0; h < 2; ++h) {
+        const v8bf kop = __builtin_bit_cast(
+            v8bf, *reinterpret_cast<const v8s*>(K + h * (P * 2 * D) + (kop_at ^ (64u * s))));
+        st[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kop, qlo, st[h], 0, 0, 0);
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const v8bf kop = __builtin_bit_cast(
-              v8bf, *reinterpret_cast<const v8s*>(K + h * (P * 2 * D) + (kop_at ^ (64u * s))));
-          st[t][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kop, qlo, st[t][h], 0, 0, 0);
-#pragma unroll
-          for (int term = 1; term >= 0; --term) {
-            st[t][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                kop, __builtin_bit_cast(v8bf, qv[t][term][s]), st[t][h], 0, 0, 0);
-          }
+        for (int term = 1; term >= 0; --term) {
+          st[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              kop, __builtin_bit_cast(v8bf, qv[term][s]), st[h], 0, 0, 0);
         }
       }
     }
     __builtin_amdgcn_s_setprio(0);
-    float p[RT][8];  // p[t][4 h + i]: key 16 h + 4 grp + i
+    float p[8];  // p[4 h + i]: key 16 h + 4 grp + i
     const bool full = (n + 1) * kBKeys <= min(key_end, hist + pos0 + 1);
     auto softmax = [&](auto full_tag) {
       constexpr bool FULL = decltype(full_tag)::value;
+      float x[8];
+      bool vis[8];
 #pragma unroll
-      for (int t = 0; t < RT; ++t) {
-        float x[8];
-        bool vis[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const int key = n * kBKeys + 16 * (j >> 2) + 4 * grp + (j & 3);
-          vis[j] = FULL || (key < key_end && (key < hist || key - hist <= qpos[t]));
-          x[j] = vis[j] ? st[t][j >> 2][j & 3] : -INFINITY;
-        }
-        const float mx = row_max(fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])),
-                                       fmaxf(fmaxf(x[4], x[5]), fmaxf(x[6], x[7]))));
-        const float mn = fmaxf(m[t], mx);
-        // Branch-free rescale (alpha is 1 for rows whose maximum held).
-        const float alpha = exp2_ratio(m[t], mn);
-#pragma unroll
-        for (int dt = 0; dt < 8; ++dt) o[t][dt] *= alpha;
-        if (FULL && __ballot(!(fabsf(mn) < INFINITY)) == 0) {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) p[t][j] = __builtin_amdgcn_exp2f(x[j] - mn);
-        } else {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) p[t][j] = vis[j] ? exp2_ratio(x[j], mn) : 0.f;
-        }
-        // The lane's own keys; the row's four lanes are added at the end.
-        l[t] = l[t] * alpha + (((p[t][0] + p[t][1]) + (p[t][2] + p[t][3])) +
-                               ((p[t][4] + p[t][5]) + (p[t][6] + p[t][7])));
-        m[t] = mn;
+      for (int j = 0; j < 8; ++j) {
+        const int key = n * kBKeys + 16 * (j >> 2) + 4 * grp + (j & 3);
+        vis[j] = FULL || (key < key_end && (key < hist || key - hist <= qpos));
+        x[j] = vis[j] ? st[j >> 2][j & 3] : -INFINITY;
       }
+      const float mx = row_max(fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])),
+                                     fmaxf(fmaxf(x[4], x[5]), fmaxf(x[6], x[7]))));
+      const float mn = fmaxf(m, mx);
+      // Branch-free rescale (alpha is 1 for rows whose maximum held).
+      const float alpha = exp2_ratio(m, mn);
+#pragma unroll
+      for (int dt = 0; dt < 8; ++dt) o[dt] *= alpha;
+      if (FULL && __ballot(!(fabsf(mn) < INFINITY)) == 0) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) p[j] = __builtin_amdgcn_exp2f(x[j] - mn);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) p[j] = vis[j] ? exp2_ratio(x[j], mn) : 0.f;
+      }
+      // The lane's own keys; the row's four lanes are added at the end.
+      l = l * alpha + (((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7])));
+      m = mn;
     };
     if (full) {
       softmax(std::true_type{});
@@ -460,17 +439,14 @@ __device__ __forceinline__ void prefill_body_bmma(PrefillKernelArgs a,
       // O^T += V^T P^T: A = V^T rows (dims 16 dt + col) at contraction
       // indices 8 grp .. + 7, B = the lane's own 8 probabilities of row col
       // in the same order, as three bf16 terms.
-      v8s pv[RT][3];
+      v8s pv[3];
 #pragma unroll
-      for (int t = 0; t < RT; ++t) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          short h, mm, lo;
-          split3_prob(p[t][j], h, mm, lo);
-          pv[t][0][j] = h;
-          pv[t][1][j] = mm;
-          pv[t][2][j] = lo;
-        }
+      for (int j = 0; j < 8; ++j) {
+        short h, mm, lo;
+        split3_prob(p[j], h, mm, lo);
+        pv[0][j] = h;
+        pv[1][j] = mm;
+        pv[2][j] = lo;
       }
       __builtin_amdgcn_s_setprio(1);
 #pragma unroll
@@ -482,12 +458,9 @@ __device__ __forceinline__ void prefill_body_bmma(PrefillKernelArgs a,
         const v8bf vop = __builtin_bit_cast(
             v8bf, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
 #pragma unroll
-        for (int t = 0; t < RT; ++t) {
-#pragma unroll
-          for (int term = 2; term >= 0; --term) {
-            o[t][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                vop, __builtin_bit_cast(v8bf, pv[t][term]), o[t][dt], 0, 0, 0);
-          }
+        for (int term = 2; term >= 0; --term) {
+          o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              vop, __builtin_bit_cast(v8bf, pv[term]), o[dt], 0, 0, 0);
         }
       }
     }
@@ -498,31 +471,24 @@ __device__ __forceinline__ void prefill_body_bmma(PrefillKernelArgs a,
   }
 
   bool nan_row = false;
+  l = row_sum(l);
+  nan_row = nan_row || !(l < INFINITY);  // NaN, or a sum that overflowed
 #pragma unroll
-  for (int t = 0; t < RT; ++t) {
-    l[t] = row_sum(l[t]);
-    nan_row = nan_row || !(l[t] < INFINITY);  // NaN, or a sum that overflowed
+  for (int dt = 0; dt < 8; ++dt)
 #pragma unroll
-    for (int dt = 0; dt < 8; ++dt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) nan_row = nan_row || isnan(o[t][dt][i]);
-  }
+    for (int i = 0; i < 4; ++i) nan_row = nan_row || isnan(o[dt][i]);
   if (__ballot(nan_row) != 0 && lane == 0) s_redo = 1;
   const int any_bad = __syncthreads_or(bad);
   if (tid == 0) redo[block] = s_redo != 0 ? 1u : 0u;
   const float vscale = FP8 ? a.v_scale : 1.0f;
+  if (qpos >= T) return;
+  const bool no_result = any_bad || m == -INFINITY;
+  const float inv = no_result ? NAN : vscale / l;
 #pragma unroll
-  for (int t = 0; t < RT; ++t) {
-    if (qpos[t] >= T) continue;
-    const bool nan_row = any_bad || m[t] == -INFINITY;
-    const float inv = nan_row ? NAN : vscale / l[t];
-#pragma unroll
-    for (int dt = 0; dt < 8; ++dt) {
-      float4 r = make_float4(o[t][dt][0] * inv, o[t][dt][1] * inv, o[t][dt][2] * inv,
-                             o[t][dt][3] * inv);
-      if (nan_row) r = make_float4(NAN, NAN, NAN, NAN);
-      *reinterpret_cast<float4*>(a.out + qrow[t] + 16 * dt + 4 * grp) = r;
-    }
+  for (int dt = 0; dt < 8; ++dt) {
+    float4 r = make_float4(o[dt][0] * inv, o[dt][1] * inv, o[dt][2] * inv, o[dt][3] * inv);
+    if (no_result) r = make_float4(NAN, NAN, NAN, NAN);
+    *reinterpret_cast<float4*>(a.out + qrow + 16 * dt + 4 * grp) = r;
   }
 }
 

@@ -181,10 +181,12 @@ def test_decode_steps_match_oracle_on_rounded_values(device, hq, fused):
     batch.close()
 
 
-def test_cascade_decode_on_bf16_pages(device):
+@pytest.mark.parametrize("HQ", [16, 32])
+def test_cascade_decode_on_bf16_pages(device, HQ):
     """Forks of one prompt share its pages; the decode step attends them once
-    (cascade prefix pass, bf16 staging) plus each fork's own pages."""
-    L, H, HQ = 1, 4, 16
+    (cascade prefix pass with bf16 staging: the fused launch at G 4, the side
+    stream beside the matrix-core decode at G 8) plus each fork's own pages."""
+    L, H = 1, 4
     rng = np.random.default_rng(21)
     N = 64
     cache = hx.PagedKvCache(L, H, D, P, N, page_dtype="bf16")

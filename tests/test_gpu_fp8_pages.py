@@ -231,11 +231,11 @@ def test_decode_steps_match_oracle_on_rounded_values(device, hq, fused):
 @pytest.mark.parametrize("hq", [8, 32])
 def test_decode_over_many_short_units_matches_oracle(device, hq):
     """1024 sequences of 0-40 tokens (a quarter of them empty, so their
-    unit is the tail alone): each stream wavefront runs through several
-    one- and two-page units in a row, so the query rows of up to three units
-    are in LDS at once (one being attended, two loading) and every area is
-    reused many times (about 16 K pages over the 4096 fp8 stream wavefronts
-    of a 256-CU GPU: four pages each)."""
+    unit is the tail alone): each wavefront runs through several one- to
+    four-page units in a row, with the next unit's query rows fetched beside
+    its first page or, where the unit before has one page here, after it
+    (about 19 K pages over the 3072 fp8 wavefronts of a 256-CU GPU: seven
+    each)."""
     L, H, B = 1, 8, 1024
     rng = np.random.default_rng(29 + hq)
     lengths = rng.integers(0, 41, size=B)
