@@ -22,7 +22,7 @@
 // over 1024 keys: 390 us before, 27 us now; one row of the same 143 -> 23 us;
 // 16/4 heads of 96 dims, 160 rows over 1660 keys 2.0 ms -> 66 us.  A call of
 // a few keys is a chain of latencies: 4 heads of 16 dims over 65 keys 8.0 us for
-// the scalar kernel, 8.2 with the scores through the workspace, 5.8 as it is
+// the scalar kernel, 8.2 with the scores through the workspace, 5.6 as it is
 // (kernel alone).
 #include "kernels.hpp"
 
@@ -42,12 +42,31 @@ using prefill_detail::row_max;
 using prefill_detail::row_sum;
 using prefill_detail::v4f;
 
+// Division by a value fixed for the launch, of 0 <= n < 2^31: multiplication
+// by 2^(31 + l) / d rounded up, l = ceil(log2 d), which is exact there (T.
+// Granlund and P. Montgomery, 1994).  The compiler's division is a chain of
+// dozens of instructions, of which a call of a few keys ran several in a row
+// before its first load.
+struct Divisor {
+  unsigned factor;
+  int shift;
+  __device__ __forceinline__ int operator()(int n) const {
+    return static_cast<int>(static_cast<unsigned long long>(factor) * static_cast<unsigned>(n) >>
+                            shift);
+  }
+};
+Divisor divisor(std::size_t d) {  // 1 <= d < 2^31
+  int l = 0;
+  while ((std::size_t{1} << l) < d) ++l;
+  return Divisor{static_cast<unsigned>(((1ull << (31 + l)) + d - 1) / d), 31 + l};
+}
+
 struct TiledArgs {
   GenericArgs g;
   int key_dim, value_dim, block_tokens, history, tail, keys, queries, rows, offset;
   bool quad;    // history is a multiple of 4
   bool vec_ws;  // workspace rows are 16-byte aligned
-  int block_shift;  // log2 of block_tokens, or -1
+  Divisor by_block, by_queries, by_vectors;  // block_tokens, queries, value vectors
   float qscale;  // 1 / sqrt(key_dim); scores of calls past HELD also times log2(e)
 };
 
@@ -117,10 +136,7 @@ __global__ __launch_bounds__(tiled_waves<DM>() * 64) void tiled_attention_kernel
   const int kvh = static_cast<int>(blockIdx.y);
   const int heads = static_cast<int>(a.g.q_heads / a.g.kv_heads);
   const int T = a.queries;
-  // Division by the query count and the page size: a chain of dozens of
-  // instructions each, which the usual one row and power of two spare.
-  auto by_queries = [&](int x) { return T == 1 ? x : x / T; };
-  auto row_of = [&](int x) { return T == 1 ? 0 : x % T; };
+  auto row_of = [&](int x) { return x - a.by_queries(x) * T; };
   const int r0 = static_cast<int>(blockIdx.x) * 16;
   const int r1 = min(r0 + 16, a.rows) - 1;
 
@@ -128,11 +144,11 @@ __global__ __launch_bounds__(tiled_waves<DM>() * 64) void tiled_attention_kernel
   const bool live = r0 + col < a.rows;
   const int r = live ? r0 + col : r1;
   const int t = row_of(r);
-  const std::size_t qrow = (static_cast<std::size_t>(kvh) * heads + by_queries(r)) * T + t;
+  const std::size_t qrow = (static_cast<std::size_t>(kvh) * heads + a.by_queries(r)) * T + t;
   const int qpos = a.offset + t;
   // Keys below `all` are seen by every row of the tile, keys from `seen` on
   // by none.
-  const bool one_head = by_queries(r0) == by_queries(r1);
+  const bool one_head = a.by_queries(r0) == a.by_queries(r1);
   const int all = min(a.keys, a.offset + (one_head ? row_of(r0) : 0) + 1);
   const int seen = min(a.keys, a.offset + (one_head ? row_of(r1) : T - 1) + 1);
   float* const srow = a.g.workspace + qrow * static_cast<std::size_t>(a.keys);
@@ -155,7 +171,7 @@ __global__ __launch_bounds__(tiled_waves<DM>() * 64) void tiled_attention_kernel
     bad = false;
     if (key >= seen) return -1;
     if (key >= a.history) return -2 - (static_cast<long long>(kvh) * a.tail + (key - a.history));
-    const int page = a.block_shift >= 0 ? key >> a.block_shift : key / a.block_tokens;
+    const int page = a.by_block(key);
     const std::uint32_t phys = a.g.table[page];
     if (phys >= a.g.physical_blocks) {
       bad = true;
@@ -353,7 +369,7 @@ __global__ __launch_bounds__(tiled_waves<DM>() * 64) void tiled_attention_kernel
   __syncthreads();
   const int vectors = (a.value_dim + 3) / 4;
   for (int e = static_cast<int>(threadIdx.x); e < 16 * vectors; e += static_cast<int>(blockDim.x)) {
-    const int rr = e / vectors;
+    const int rr = a.by_vectors(e);
     const int d = (e - rr * vectors) * 4;
     if (r0 + rr > r1) continue;
     float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -370,7 +386,7 @@ __global__ __launch_bounds__(tiled_waves<DM>() * 64) void tiled_attention_kernel
     const int rt = r0 + rr;
     float* const dst =
         a.g.out +
-        ((static_cast<std::size_t>(kvh) * heads + by_queries(rt)) * T + row_of(rt)) * a.value_dim + d;
+        ((static_cast<std::size_t>(kvh) * heads + a.by_queries(rt)) * T + row_of(rt)) * a.value_dim + d;
     if constexpr (VEC) {
       *reinterpret_cast<float4*>(dst) = make_float4(o.x * inv, o.y * inv, o.z * inv, o.w * inv);
     } else {
@@ -459,7 +475,9 @@ hipError_t launch_tiled_attention(const GenericArgs& a, hipStream_t stream) {
   k.offset = static_cast<int>(a.offset);
   k.quad = a.history % 4 == 0;
   k.vec_ws = (a.history + a.tail) % 4 == 0 && aligned(a.workspace);
-  k.block_shift = (a.block_tokens & (a.block_tokens - 1)) == 0 ? __builtin_ctzll(a.block_tokens) : -1;
+  k.by_block = divisor(a.block_tokens);
+  k.by_queries = divisor(a.queries);
+  k.by_vectors = divisor((a.value_dim + 3) / 4);
   const bool vec = a.key_dim % 4 == 0 && a.value_dim % 4 == 0 && aligned(a.query) &&
                    aligned(a.key_blocks) && aligned(a.value_blocks) && aligned(a.tail_key) &&
                    aligned(a.tail_value) && aligned(a.out);
