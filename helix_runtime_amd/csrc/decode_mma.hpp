@@ -8,10 +8,10 @@
 // products of 4 query heads, the widening, the cross-lane score reduction),
 // which takes longer than a reduced-precision page's bytes do.  Here both
 // products run on the matrix cores and a page costs about 130 vector and 12
-// matrix instructions.  64 sequences of 512-8192 tokens, 32/8 heads, one
-// layer: fp8 pages 103-110 -> 64-66 us for this kernel (384 MB, 5.9 TB/s),
-// bf16 pages 118 -> 115 us (766 MB, 6.65 TB/s, the page-read rate of this
-// part; those were bound by HBM before as well).
+// matrix instructions.  64 sequences of 512-8192 tokens, 32/8 heads, one layer
+// with its merge: fp8 pages 111 -> 70 us (347 MB, 4.9 TB/s), bf16 pages 125 ->
+// 120 us (692 MB, 5.8 TB/s); a loads-only read of pages moves 6.6 TB/s, the
+// launch's start, its end and the merge are the rest.
 //
 // Exactness.  A bf16 page value is exact in bf16, and so is the bare code
 // value of an fp8 element (the key scale is part of qscale, the value scale
@@ -32,21 +32,23 @@
 // transposed on the way out of LDS (ds_read_b64_tr_b16 / _b8), each lane
 // getting the 4 keys of one dim whose probabilities the score tile left it.
 //
-// Shape, measured on the fp8 pages above (whole layer with the merge, us):
-// three wavefronts per SIMD 72, four 75-99 (spills, and one more partial per
-// wavefront for the merge), two 73; a stage of two pages (whose P.V runs on
-// the K = 32 instruction) with two wavefronts 77-80; three and four stages
-// 76-80.  bf16 pages: two wavefronts per SIMD (LDS: 18 KB each) 120, one
-// with two-page stages 123.
+// Shape, measured on the fp8 pages above (whole layer with the merge, us, at
+// the time against 72 for this form): three wavefronts per SIMD 72, four 75-99
+// (spills, and one more partial per wavefront for the merge; 80 now), two 73;
+// a stage of two pages (whose P.V runs on the K = 32 instruction) with two
+// wavefronts 77-80; three and four stages 76-80; a second query area, so that
+// a unit's rows always come with its first page, 0-1 % less on units of a few
+// pages and none here.  bf16 pages: two wavefronts per SIMD (LDS: 18 KB each)
+// 120, one with two-page stages 123.
 //
 // The page descriptors (unit, physical page, visible tokens) of 64 pages are
 // formed at once, one per lane, and read back with v_readlane: no scalar
 // load or division stands between a page and the next one's loads.
 //
-// Special values.  A finite element times the three terms sums to what it
-// gives in one product, and a NaN or an infinite operand of the split stays
-// one in its high term: fp8 pages, which hold no infinities, need nothing
-// more.  A bf16 page's infinity times a term that is zero is a NaN that fp32
+// Special values.  The three terms of a finite operand times a finite element
+// add up to their product; a NaN stays one in every term, and an infinite
+// operand is its high term with zeros beside it: fp8 pages, which hold no
+// infinities, need nothing more.  A bf16 page's infinity times a term that is zero is a NaN that fp32
 // does not give.  Every such NaN reaches the range's sum or outputs, so a
 // range of bf16 pages that ends with a NaN there is scanned for infinities
 // and, if it has one, computed again with fp32 arithmetic before it is

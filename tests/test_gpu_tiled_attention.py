@@ -1,9 +1,8 @@
 """Reference-shaped attention on the fp32 matrix cores (head sizes other than
 128, other page sizes): edges of the 16-row and 16-key tiles, as many key
-tiles as wavefronts and one more, head sizes
-around the 16-, 64-, 128- and 256-dim groups and not multiples of 4, grouped
-heads, key and value sizes that differ, both entry points, unaligned tensors,
-special values.
+tiles as wavefronts and one more, head sizes around the 16-, 64-, 128- and
+256-dim groups and not multiples of 4, grouped heads, key and value sizes that
+differ, both entry points, unaligned tensors, special values.
 
 Reference: 64-bit numpy for finite inputs (max-abs 2e-5 plus rel 1e-4 on
 outputs, 2e-6 on probabilities, the contract of the reference-shaped entry),
