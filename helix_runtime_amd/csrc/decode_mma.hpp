@@ -46,16 +46,15 @@
 // load or division stands between a page and the next one's loads.
 //
 // Special values.  The three terms of a finite operand times a finite element
-// add up to their product; a NaN stays one in every term, and an infinite
-// operand is its high term with zeros beside it: fp8 pages, which hold no
-// infinities, need nothing more.  A bf16 page's infinity times a term that is zero is a NaN that fp32
-// does not give.  Every such NaN reaches the range's sum or outputs, so a
-// range of bf16 pages that ends with a NaN there is scanned for infinities
-// and, if it has one, computed again with fp32 arithmetic before it is
-// published.  One layer of the 64 sequences above, one of them with a NaN
-// element: bf16 pages 119 -> 122 us, fp8 pages 72 -> 73 (1100 and 730 when
-// every such range was computed again, row by row); with an infinite key,
-// bf16 pages 201 us.
+// add up to their product, and a NaN or infinite operand is its high term with
+// zeros beside it: fp8 pages, which hold no infinities, need nothing more.  A
+// bf16 page's infinity times a term that is zero is a NaN that fp32 does not
+// give.  Every such NaN reaches the range's sum or outputs, so a range of bf16
+// pages that ends with a NaN there is scanned for infinities and, if it has
+// one, computed again with fp32 arithmetic before it is published.  One layer
+// of the 64 sequences above, one of them with a NaN element: bf16 pages 119 ->
+// 122 us, fp8 pages 72 -> 73 (1100 and 730 when every such range was computed
+// again, row by row); with an infinite key, bf16 pages 201 us.
 #pragma once
 
 #include "bf16.hpp"
