@@ -84,3 +84,46 @@ def test_known_lengths_match_oracle(device, hkv, group, batch, tokens):
     np.testing.assert_allclose(out.cpu().numpy(), ref, atol=ATOL, rtol=RTOL)
     batch_.close()
     cache.close()
+
+
+@pytest.mark.parametrize("dtype", ["f32", "fp8"])
+@pytest.mark.parametrize("hkv,group", [(8, 4), (32, 1)])
+def test_captured_layer_replays_at_grown_lengths(device, dtype, hkv, group):
+    """A layer captured where every unit has few partials, replayed after one
+    sequence has grown to hundreds: the launch shape stays, the result follows."""
+    gen = torch.Generator(device=device)
+    gen.manual_seed(hkv)
+    r = lambda *s: torch.randn(*s, device=device, generator=gen)  # noqa: E731
+    more = dict(k_scale=0.03, v_scale=0.015) if dtype == "fp8" else {}
+    cache = hx.PagedKvCache(1, hkv, D, P, 700, page_dtype=dtype, **more)
+    seqs = [cache.create_sequence() for _ in range(4)]
+    for s in seqs:
+        cache.append_layer_major(s, [r(hkv, 98, D)], [r(hkv, 98, D)])
+    batch = hx.DecodeBatch(cache, seqs, hkv * group, max_tokens=9000)
+    q, tk, tv = r(4, hkv * group, D), r(4, hkv, D), r(4, hkv, D)
+    got, want = torch.empty_like(q), torch.empty_like(q)
+    stream = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        batch.prepare()
+        batch.attention_layer(0, q, tk, tv, want)
+        stream.synchronize()
+        with torch.cuda.graph(graph, stream=stream):
+            batch.attention_layer(0, q, tk, tv, got)
+        for grown in (0, 1, 2500, 5000):
+            if grown:
+                batch.append_layer(0, tk, tv)
+                k, v = r(hkv, grown, D), r(hkv, grown, D)
+                stream.synchronize()
+                cache.append_layer_major(seqs[1], [k], [v])
+                batch.prepare()
+            for _ in range(2):
+                got.fill_(7.0)
+                graph.replay()
+                batch.attention_layer(0, q, tk, tv, want)
+                stream.synchronize()
+                np.testing.assert_allclose(got.cpu().numpy(), want.cpu().numpy(), atol=ATOL, rtol=RTOL)
+    assert torch.isfinite(want).all()
+    batch.close()
+    cache.close()
