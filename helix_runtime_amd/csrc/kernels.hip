@@ -2665,9 +2665,12 @@ void launch_merge_variant(unsigned units, hipStream_t stream, const DecodeKernel
 // per unit a half-wavefront leaves the other half empty, so two cost no
 // dispatch: better at few rows and with many partials (32/32 heads, 8 of 98
 // tokens 13.9 with 1, 13.7 with 2; 128, one of 8000 among 100s, 126.2, 123.5),
-// worse where a full launch has few (32 of 60: 18.9, 19.2).
+// worse where a full launch has few (32 of 60: 18.9, 19.2).  From 4096 rows on
+// more lanes cost every launch whose lengths are not known to be ragged; known
+// ones (`known`) with more than 16 partials in a unit get 4.
 template <int G>
-void launch_stream_merge_group(hipStream_t stream, const DecodeKernelArgs& k, std::size_t most) {
+void launch_stream_merge_group(hipStream_t stream, const DecodeKernelArgs& k, std::size_t most,
+                               bool known) {
   const unsigned units = static_cast<unsigned>(k.batch) * static_cast<unsigned>(k.kv_heads);
   const unsigned rows = units * G;
   if (most <= 8) {
@@ -2676,7 +2679,7 @@ void launch_stream_merge_group(hipStream_t stream, const DecodeKernelArgs& k, st
     } else {
       launch_merge_variant<G, 1>(units, stream, k);
     }
-  } else if (rows >= 4096) {
+  } else if (rows >= 4096 && (most <= 16 || !known)) {
     launch_merge_variant<G, G == 1 ? 2 : 1>(units, stream, k);
   } else if (rows >= 2048) {
     launch_merge_variant<G, 4>(units, stream, k);
@@ -2688,12 +2691,12 @@ void launch_stream_merge_group(hipStream_t stream, const DecodeKernelArgs& k, st
 }
 
 hipError_t launch_stream_merge(std::size_t group, hipStream_t stream, const DecodeKernelArgs& k,
-                               std::size_t most) {
+                               std::size_t most, bool known) {
   switch (group) {
-    case 1: launch_stream_merge_group<1>(stream, k, most); break;
-    case 2: launch_stream_merge_group<2>(stream, k, most); break;
-    case 4: launch_stream_merge_group<4>(stream, k, most); break;
-    case 8: launch_stream_merge_group<8>(stream, k, most); break;
+    case 1: launch_stream_merge_group<1>(stream, k, most, known); break;
+    case 2: launch_stream_merge_group<2>(stream, k, most, known); break;
+    case 4: launch_stream_merge_group<4>(stream, k, most, known); break;
+    case 8: launch_stream_merge_group<8>(stream, k, most, known); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -2790,7 +2793,8 @@ hipError_t launch_decode(const DecodeArgs& a, hipStream_t stream) {
           e = hipEventRecord(a.between_event, stream);
           if (e != hipSuccess) return e;
         }
-        return launch_stream_merge(group, stream, k, most_partials(a, waves, k.prefix_chunks));
+        return launch_stream_merge(group, stream, k, most_partials(a, waves, k.prefix_chunks),
+                                   a.longest_pages != 0);
       }
       if (overlap) {
         hipError_t e = hipEventRecord(a.fork_event, stream);
@@ -2832,7 +2836,8 @@ hipError_t launch_decode(const DecodeArgs& a, hipStream_t stream) {
       e = hipStreamWaitEvent(stream, a.join_event, 0);
       if (e != hipSuccess) return e;
     }
-    return launch_stream_merge(group, stream, k, most_partials(a, waves, k.prefix_chunks));
+    return launch_stream_merge(group, stream, k, most_partials(a, waves, k.prefix_chunks),
+                                   a.longest_pages != 0);
   }
   const WorkspaceLayout lay = layout_for(a.batch, a.q_heads, a.kv_heads, max_splits);
   k.part_o = reinterpret_cast<float*>(ws + lay.part_o);

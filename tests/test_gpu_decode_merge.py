@@ -49,18 +49,20 @@ def test_ragged_batch_matches_split_kernel(device, hkv, group, batch, long):
     np.testing.assert_allclose(results[0], results[1], atol=ATOL, rtol=RTOL)
 
 
-@pytest.mark.parametrize("hkv,group,batch,tokens", [(8, 4, 1, 60), (8, 4, 40, 98), (4, 8, 64, 300),
-                                                    (32, 1, 4, 98), (32, 1, 40, 60), (16, 2, 9, 2000),
-                                                    (8, 4, 70, 700)])
-def test_known_lengths_match_oracle(device, hkv, group, batch, tokens):
-    """A batch whose table is far wider than its sequences."""
+@pytest.mark.parametrize("hkv,group,batch,tokens,short", [
+    (8, 4, 1, 60, 60), (8, 4, 40, 98, 98), (4, 8, 64, 300, 300), (32, 1, 4, 98, 98),
+    (32, 1, 40, 60, 60), (16, 2, 9, 2000, 2000), (8, 4, 70, 700, 700), (8, 4, 130, 4000, 50),
+    (32, 1, 130, 1500, 20)])
+def test_known_lengths_match_oracle(device, hkv, group, batch, tokens, short):
+    """A batch whose table is far wider than its sequences: one of `tokens`,
+    the others of about `short`."""
     rng = np.random.default_rng(tokens + batch)
-    hq, phys = hkv * group, batch * (tokens // P + 2)
+    hq, phys = hkv * group, tokens // P + 2 + batch * (short // P + 2)
     cache = hx.PagedKvCache(1, hkv, D, P, phys)
     rows = rng.standard_normal((2, hkv, tokens, D), dtype=np.float32)
     seqs, lengths = [], []
     for b in range(batch):  # the rows' first tokens, a few fewer each
-        n = tokens - b % 7
+        n = tokens if b == batch // 2 else short - b % 7
         s = cache.create_sequence()
         cache.append_layer_major(s, *([torch.from_numpy(x[:, :n].copy()).to(device)] for x in rows))
         seqs.append(s)
